@@ -93,7 +93,8 @@ int check_attn_common(const kvq_rows* q, const kvq_rows* out, int B, int Hq, int
 
 // Head dimensions 64, 128 and 256 have kernels of their own width; any other multiple of 8 up to 256
 // runs at the next width (kvq::decode_kernel_dim), for every query length: on the decode kernel, or
-// for unquantized rows past 128 dims on the head_dim-256 kernel.
+// for unquantized rows past 128 dims on the head_dim-256 kernel. Quantized rows of 96 dims have a
+// prefill kernel too (prefill_serves_96).
 bool native_dim(int D) { return D == 64 || D == 128 || D == 256; }
 
 int check_head_dim(int D, const char* what) {
@@ -388,7 +389,9 @@ int kvq_decode_attn_static(const kvq_rows* q, const kvq_qtensor* k, const kvq_qt
 
 size_t kvq_prefill_workspace_size(int B, int Hq, int Hkv, int L, int D, int S, int window) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || S <= 0 || window < 0 || Hq % Hkv) return 0;
-  if (!native_dim(D)) return kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, window);  // the decode kernel serves
+  // the decode kernel serves; where the prefill kernel does (prefill_serves_96) its splits are fitted to
+  // the same size
+  if (!native_dim(D)) return kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, window);
   if (D == 256) return kvq::wide_workspace_bytes(B, Hq, Hkv, L, D, S, window);
   const size_t n = kvq::prefill_workspace_bytes(B, Hq, Hkv, L, D, S, window, 8);
   if (D == 64) {  // the unquantized cache at head_dim 64 runs through wide.hip's kernel
@@ -409,6 +412,20 @@ static int check_prefill_sb(const kvq_qtensor* k, const kvq_qtensor* v, int D, i
   return KVQ_OK;
 }
 
+// Whether a quantized head_dim-96 prefill call runs on the prefill kernel. A decode pass serves 4 query
+// rows (group 32) and its time grows with them, the prefill kernel's is flat up to a row block of 256:
+// 8 KV heads, 8 bits, 64 rows (16 decode passes) 14.8 us against 21.7 at 2048 keys, 38.5 against 48.1
+// at 8192 and 130 against 155 at 32768, 48 rows of 12 passes up to even; a 1999-token prompt of 32 heads
+// 1276 us on the decode kernel, 53 on the prefill kernel. So the line is at 64 rows. The calls that
+// the prefill kernel cannot take as the decode kernel does stay there too: output rows that are not
+// 16-byte aligned, and a bf16 cache without range words, whose values may leave the fp16 operands.
+static bool prefill_serves_96(const kvq_qtensor* k, const kvq_qtensor* v, const kvq_rows* out, int Hq, int Hkv, int L,
+                              int D, int dtype) {
+  if (D != 96 || (int64_t)(Hq / Hkv) * L <= 64) return false;
+  if (dtype == KVQ_DTYPE_BF16 && (!k->range_exp || !v->range_exp)) return false;
+  return aligned(out->data, 16) && !((out->stride_b | out->stride_h | out->stride_l) % 8);
+}
+
 int kvq_prefill_attn(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const int32_t* seq_lens,
                      const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int bits, int group_size,
                      int dtype, float scale, int causal, int window, void* workspace, size_t workspace_bytes,
@@ -417,7 +434,8 @@ int kvq_prefill_attn(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor*
   int rc = check_attn(q, k, v, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale, window,
                       kvq_prefill_workspace_size(B, Hq, Hkv, L, D, S, window), workspace, workspace_bytes);
   if (rc) return rc;
-  if (!native_dim(D))
+  const bool at96 = prefill_serves_96(k, v, out, Hq, Hkv, L, D, dtype);
+  if (!native_dim(D) && !at96)
     return hip_status(kvq::launch_decode(q, k, v, seq_lens, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale,
                                          causal, window, workspace, (hipStream_t)stream),
                       "prefill_attn launch (the decode kernel, head_dim other than 64/128/256)");
@@ -426,9 +444,10 @@ int kvq_prefill_attn(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor*
                                        window, workspace, (hipStream_t)stream),
                       "prefill_attn launch (head_dim 256)");
   if ((rc = check_rows(out, "out", D, true))) return rc;  // rows are stored 16 bytes at a time
-  if ((rc = check_prefill_sb(k, v, D, group_size))) return rc;
+  if (!at96 && (rc = check_prefill_sb(k, v, D, group_size))) return rc;
   return hip_status(kvq::launch_prefill(q, k, v, seq_lens, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale,
-                                        causal, window, workspace, (hipStream_t)stream),
+                                        causal, window, workspace,
+                                        kvq_prefill_workspace_size(B, Hq, Hkv, L, D, S, window), (hipStream_t)stream),
                     "prefill_attn launch");
 }
 
@@ -476,7 +495,8 @@ int kvq_paged_prefill_attn(const kvq_rows* q, const kvq_qtensor* k_pool, const k
                             group_size, dtype, scale, window, kvq_prefill_workspace_size(B, Hq, Hkv, L, D, S, window),
                             workspace, workspace_bytes);
   if (rc) return rc;
-  if (!native_dim(D))
+  const bool at96 = prefill_serves_96(k_pool, v_pool, out, Hq, Hkv, L, D, dtype);
+  if (!native_dim(D) && !at96)
     return hip_status(kvq::launch_decode_paged(q, k_pool, v_pool, num_pages, block_table, table_stride, seq_lens, out,
                                                B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale, causal, window,
                                                workspace, (hipStream_t)stream),
@@ -487,10 +507,11 @@ int kvq_paged_prefill_attn(const kvq_rows* q, const kvq_qtensor* k_pool, const k
                                              (hipStream_t)stream),
                       "paged_prefill_attn launch (head_dim 256)");
   if ((rc = check_rows(out, "out", D, true))) return rc;  // rows are stored 16 bytes at a time
-  if ((rc = check_prefill_sb(k_pool, v_pool, D, group_size))) return rc;
+  if (!at96 && (rc = check_prefill_sb(k_pool, v_pool, D, group_size))) return rc;
   return hip_status(kvq::launch_prefill_paged(q, k_pool, v_pool, num_pages, block_table, table_stride, seq_lens, out, B,
                                               Hq, Hkv, L, D, S, bits, group_size, dtype, scale, causal, window,
-                                              workspace, (hipStream_t)stream),
+                                              workspace, kvq_prefill_workspace_size(B, Hq, Hkv, L, D, S, window),
+                                              (hipStream_t)stream),
                     "paged_prefill_attn launch");
 }
 

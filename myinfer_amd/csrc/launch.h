@@ -41,13 +41,16 @@ hipError_t launch_decode_dense(const kvq_rows* q, const kvq_rows* k, const kvq_r
                                const kvq_mask* mask = nullptr);
 
 size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window, int bits);
+// workspace_bytes: what the call's shapes entitle it to (kvq_prefill_workspace_size), which bounds the
+// key splits; not the size of the caller's buffer, so that a call's splits follow from its shapes
 hipError_t launch_prefill(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const int32_t* seq_lens,
                           const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype,
-                          float scale, int causal, int window, void* workspace, hipStream_t stream);
+                          float scale, int causal, int window, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream);
 hipError_t launch_prefill_paged(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, int num_pages,
                                 const int32_t* table, int64_t table_stride, const int32_t* seq_lens, const kvq_rows* out,
                                 int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype, float scale,
-                                int causal, int window, void* workspace, hipStream_t stream);
+                                int causal, int window, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // wide.hip: head_dim 256 over quantized (4/8 bits, groups 64/128) and unquantized caches, and head_dim 64
 // over unquantized caches, any query length
 size_t wide_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window);

@@ -7,7 +7,7 @@
 // with query l at position S_b - L + l, keys <= position when causal, keys > position - window
 // when a sliding window is set.
 //
-// Design (head_dim D = 128 or 64, 64-key tiles, a workgroup = 8 waves = 256 query rows, one per CU):
+// Design (head_dim D = 128, 96 or 64, 64-key tiles, a workgroup = 8 waves = 256 query rows, one per CU):
 //  * A workgroup serves 256 consecutive rows of one (sequence, KV head) in position-major order
 //    (row = position * rep + local head), so all rep query heads of a position share each K/V
 //    tile and a causal boundary cuts only a few positions.
@@ -57,48 +57,72 @@ constexpr int kRawSlots = 3;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 
 // The raw tile ring. A slot holds one 64-key tile as loaded: [K codes][V codes][sK, bK, sV, bV],
-// code rows with their 16-byte chunks XOR-swizzled by row (chunk c of row r at position
-// c ^ swz(r)), each scale/bias array as 64 PC 4-byte cells: with NG = D / G >= 2 scale groups
-// per row, cell PC key + c holds groups 2c and 2c + 1 of the key (PC = NG / 2); with one group,
-// cell key holds it in its low half (PC = 1).
+// code rows with their 16-byte chunks permuted by row (chunk c of row r at position pos(r, c)), each
+// scale/bias array as 64 PC 4-byte cells: with an even number NG = D / G of scale groups per row,
+// cell PC key + c holds groups 2c and 2c + 1 of the key (PC = NG / 2); with an odd number, cell
+// NG key + g holds group g in its low half (PC = NG; the rows are then only 2-byte aligned).
 // BITS == 16 is the unquantized cache: raw T rows, no scales or biases.
 template <int BITS, int G = 64, int D = 128>
 struct RawCfg {
   static constexpr bool DENSE = BITS == 16;
   static_assert(G == 32 || G == 64 || G == 128, "group sizes 32, 64, 128");
-  static_assert(D == 128 || (D == 64 && !DENSE), "head_dim 128, or 64 for quantized caches");
-  static_assert(G <= D, "a group lies in one row");
+  static_assert(D == 128 || (D == 64 && !DENSE) || (D == 96 && G == 32 && !DENSE),
+                "head_dim 128, or 64 or 96 for quantized caches");
+  static_assert(G <= D && D % G == 0, "a group lies in one row");
   static constexpr int NG = D / G;                  // scale groups per key row
   static constexpr int ROWB = D * BITS / 8;         // code bytes per key row
   static constexpr int CPR = ROWB / 16;             // 16-byte chunks per row
-  static constexpr int RPI = 64 / CPR;              // rows per 1 KiB DMA instruction
-  static constexpr int CI = kPT / RPI;              // DMA instructions per K (or V) code tile
   static constexpr int KB = kPT * ROWB;             // bytes of a K (or V) code tile
-  static constexpr int PC = NG >= 2 ? NG / 2 : 1;  // 4-byte cells per key in a scale/bias array
+  static constexpr int CI = KB / 1024;              // DMA instructions per K (or V) code tile
+  static constexpr bool CELL1 = NG % 2 == 1;        // one group per scale/bias cell
+  static constexpr int PC = CELL1 ? NG : NG / 2;    // 4-byte cells per key in a scale/bias array
   static constexpr int SBB = DENSE ? 0 : 256 * PC;  // bytes of one scale/bias array
   static constexpr int SLOT = 2 * KB + 4 * SBB;
-  // code DMA instructions per wave: with fewer than one per wave (4-bit, D = 64) waves 0 .. 2 CI - 1
-  // issue one each and the others none
-  static constexpr int CPW = 2 * CI >= kPW ? 2 * CI / kPW : 1;
-  static constexpr int CODE_WAVES = 2 * CI >= kPW ? kPW : 2 * CI;
+  // the waves that dequantize: V^T in waves [0, NSW), K in [NSW, 2 NSW) (256 threads each for
+  // D = 128, 192 for D = 96, 128 for D = 64); the other waves only compute
+  static constexpr int NSW = D / 32;
+  // code DMA instructions per wave: when the 2 CI of a tile do not divide over the 8 waves (D = 96, or
+  // 4-bit D = 64) the dequantizing waves issue them and the others none
+  static constexpr int CODE_WAVES = (2 * CI) % kPW == 0 ? kPW : 2 * NSW;
+  static constexpr int CPW = 2 * CI / CODE_WAVES;
   // The chunk swizzle of row r. Quantized tiles fold in r / 16: the V^T staging reads one dim
   // quad of 8 keys per lane, and keys 16 apart (the same key % CPR) would otherwise share LDS
   // banks (a 4-way conflict at 8 bits); this spreads them over the banks. Unquantized rows keep
   // r % CPR (their staging and operand reads index it directly).
   static __device__ __forceinline__ constexpr int swz(int r) { return (DENSE ? r : r ^ (r >> 4)) % CPR; }
-  // the waves that dequantize: V^T in waves [0, NSW), K in [NSW, 2 NSW) (256 threads each for
-  // D = 128, 128 for D = 64); the other waves only compute
-  static constexpr int NSW = D / 32;
-  // 64-cell scale/bias DMA instructions per wave: 4 PC of them fill the four arrays, one per wave
-  // (with PC = 1 two waves fill the same cells)
-  static constexpr int SBW = DENSE ? 0 : 1;
+  // Rows of 6 or 3 chunks (D = 96) rotate them by a multiple that depends on r / 16 instead: such rows
+  // are 24 or 12 banks long, so keys 4 apart already differ and only keys 16 apart would meet (the
+  // four rotations 0, 3, 5, 2 of 6 give the V^T staging's chunk pairs four starts).
+  static constexpr bool ROT = (CPR & (CPR - 1)) != 0;
+  static __device__ __forceinline__ constexpr int rot(int r) {
+    return CPR == 6 ? (0x2530 >> (4 * ((r >> 4) & 3))) & 7 : ((r >> 4) & 3) % 3;
+  }
+  // position of chunk c in row r, and the chunk at position q
+  static __device__ __forceinline__ constexpr int pos(int r, int c) {
+    return ROT ? (c + rot(r)) % CPR : c ^ swz(r);
+  }
+  static __device__ __forceinline__ constexpr int chunk_at(int r, int q) {
+    return ROT ? (q + CPR - rot(r)) % CPR : q ^ swz(r);
+  }
+  // 64-cell scale/bias DMA instructions: 4 PC of them fill the four arrays. Up to 8 they go one per
+  // wave (with PC = 1 two waves fill the same cells); the 12 of D = 96 go two to each of the six
+  // waves that load codes.
+  static constexpr int SBW = DENSE ? 0 : 4 * PC <= kPW ? 1 : 4 * PC / CODE_WAVES;
+  static constexpr bool SB_ALL = 4 * PC <= kPW;     // every wave issues them
   static constexpr int IPT = CPW + SBW;             // DMA instructions per tile of a wave that loads codes
-  static constexpr int IPT_NOCODE = SBW;            // ... and of one that does not
+  static constexpr int IPT_NOCODE = SB_ALL ? SBW : 0;  // ... and of one that does not
   static_assert(CPW * CODE_WAVES == 2 * CI, "code DMAs divide evenly over the waves that issue them");
   static_assert(CODE_WAVES >= 2 * NSW, "the dequantizing waves load codes");
-  static_assert(DENSE || 4 * PC <= kPW, "scale/bias DMAs fit one per wave");
+  static_assert(DENSE || SB_ALL || SBW * CODE_WAVES == 4 * PC, "scale/bias DMAs divide evenly");
+  // scale/bias DMA j of wave w: its array and which 64 cells of it
+  static __device__ __forceinline__ constexpr int sb_array(int w, int j) { return SB_ALL ? w / 2 : (w * SBW + j) / PC; }
+  static __device__ __forceinline__ constexpr int sb_part(int w, int j) {
+    return SB_ALL ? (w % 2) % PC : (w * SBW + j) % PC;
+  }
   // byte offset of group g of key `key` inside a scale/bias array
-  static __host__ __device__ constexpr int sb_off(int key, int g) { return 4 * (PC * key + g / 2) + 2 * (g & 1); }
+  static __host__ __device__ constexpr int sb_off(int key, int g) {
+    return CELL1 ? 4 * (PC * key + g) : 4 * (PC * key + g / 2) + 2 * (g & 1);
+  }
 };
 
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -158,9 +182,8 @@ static_assert(v_keys_split(), "slot keys are a per-lane base (low two bits clear
 
 
 // This wave's share of a raw tile: CPW 1 KiB code loads (K instructions first, then V; none for
-// waves from CODE_WAVES on) and one 64-cell scale/bias load (array wave / 2, cells 64 part .. with
-// part = (wave % 2) % PC; 4-byte cells, or 2-byte values into the low halves when PC = 1 holds a
-// single group).
+// waves from CODE_WAVES on) and SBW 64-cell scale/bias loads (array sb_array, cells from
+// 64 sb_part; 4-byte cells, or 2-byte values into the low halves when a cell holds one group).
 template <int BITS, int G = 64, int D = 128>
 struct RawShare {
   using C = RawCfg<BITS, G, D>;
@@ -178,8 +201,9 @@ struct RawShare {
       const int q = code_on ? wave * C::CPW + j : 0;
       const bool is_k = q < C::CI;
       const int i = is_k ? q : q - C::CI;
-      const int r = i * C::RPI + lane / C::CPR;
-      const int c = (lane % C::CPR) ^ C::swz(r);
+      // 16-byte cell 64 i + lane of the tile: chunk position cell % CPR of row cell / CPR
+      const int r = C::ROT ? (64 * i + lane) / C::CPR : i * (64 / C::CPR) + lane / C::CPR;
+      const int c = C::chunk_at(r, C::ROT ? (64 * i + lane) % C::CPR : lane % C::CPR);
       code_r[j] = is_k ? kr : vr;
       code_ss[j] = is_k ? p.kc_ss : p.vc_ss;
       code_vo[j] = (uint32_t)(r * code_ss[j] + 16 * c);
@@ -187,11 +211,12 @@ struct RawShare {
     }
 #pragma unroll
     for (int j = 0; j < SBN; ++j) {
-      const int li = wave * C::SBW + j, a = li / 2, part = (li % 2) % C::PC;
+      const int w = C::SB_ALL || code_on ? wave : 0;
+      const int a = C::sb_array(w, j), part = C::sb_part(w, j);
       const int cell = 64 * part + lane;  // cell cell % PC of key cell / PC
       sb_r[j] = a == 0 ? sr[0] : a == 1 ? sr[1] : a == 2 ? sr[2] : sr[3];
       sb_ss[j] = C::DENSE ? 0 : 2 * (a < 2 ? p.ksb_ss : p.vsb_ss);
-      sb_vo[j] = (uint32_t)((cell / C::PC) * sb_ss[j] + 4 * (cell % C::PC));
+      sb_vo[j] = (uint32_t)((cell / C::PC) * sb_ss[j] + (C::CELL1 ? 2 : 4) * (cell % C::PC));
       sb_lds[j] = 2 * C::KB + C::SBB * a + 256 * part;
     }
   }
@@ -201,14 +226,16 @@ struct RawShare {
 #pragma unroll
       for (int j = 0; j < C::CPW; ++j) dma_b128(code_r[j], slot + code_lds[j], code_vo[j], (uint32_t)(k0 * code_ss[j]));
     }
+    if (C::SB_ALL || code_on) {
 #pragma unroll
-    for (int j = 0; j < C::SBW; ++j) dma_sb(sb_r[j], slot + sb_lds[j], sb_vo[j], (uint32_t)(k0 * sb_ss[j]));
+      for (int j = 0; j < C::SBW; ++j) dma_sb(sb_r[j], slot + sb_lds[j], sb_vo[j], (uint32_t)(k0 * sb_ss[j]));
+    }
   }
   static __device__ __forceinline__ void dma_sb(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t vo, uint32_t so) {
-    if constexpr (C::NG >= 2) {
-      dma_b32(r, lds, vo, so);
-    } else {
+    if constexpr (C::CELL1) {
       dma_b16(r, lds, vo, so);
+    } else {
+      dma_b32(r, lds, vo, so);
     }
   }
 
@@ -225,7 +252,7 @@ struct RawShare {
     }
 #pragma unroll
     for (int j = 0; j < SBN; ++j) {
-      const int a = (wave * C::SBW + j) / 2;
+      const int a = C::sb_array(C::SB_ALL || code_on ? wave : 0, j);
       const uint16_t* arr = a == 0 ? p.ks : a == 1 ? p.kb : a == 2 ? p.vs : p.vb;
       sb_base[j] = (const uint8_t*)(arr + (int64_t)kvh * (a < 2 ? p.ksb_sh : p.vsb_sh));
       sb_ps[j] = 2 * (a < 2 ? p.ksb_sb : p.vsb_sb);
@@ -239,10 +266,12 @@ struct RawShare {
         dma_b128(make_rsrc(code_base[j] + (int64_t)pg * code_ps[j], (uint32_t)(nv * code_ss[j])), slot + code_lds[j],
                  code_vo[j], 0u);
     }
+    if (C::SB_ALL || code_on) {
 #pragma unroll
-    for (int j = 0; j < C::SBW; ++j)
-      dma_sb(make_rsrc(sb_base[j] + (int64_t)pg * sb_ps[j], (uint32_t)(nv * sb_ss[j])), slot + sb_lds[j], sb_vo[j],
-             0u);
+      for (int j = 0; j < C::SBW; ++j)
+        dma_sb(make_rsrc(sb_base[j] + (int64_t)pg * sb_ps[j], (uint32_t)(nv * sb_ss[j])), slot + sb_lds[j], sb_vo[j],
+               0u);
+    }
   }
 };
 
@@ -322,11 +351,13 @@ __device__ __forceinline__ void stage_v(const uint8_t* raw, _Float16* vlds, cons
   for (int i = 0; i < 8; ++i) {
     const int ko = v_key_offset(i);
     const int sw = (((kb % C::CPR) | (i & 3)) ^ (kb >> 4)) % C::CPR;
+    // (rotated rows depend on key >> 4 alone: one address per lane)
+    auto at = [&](int c) { return C::ROT ? C::pos(kb, c) : c ^ sw; };
     uint32_t bytes;  // codes of dims 4 d4 .. 4 d4 + 3 as 4 bytes
     if constexpr (BITS == 8) {
-      bytes = *(const uint32_t*)(vr + ko * C::ROWB + 16 * ((d4 >> 2) ^ sw) + 4 * (d4 & 3));
+      bytes = *(const uint32_t*)(vr + ko * C::ROWB + 16 * at(d4 >> 2) + 4 * (d4 & 3));
     } else {
-      const uint32_t h = *(const uint16_t*)(vr + ko * C::ROWB + 16 * ((d4 >> 3) ^ sw) + 2 * (d4 & 7));
+      const uint32_t h = *(const uint16_t*)(vr + ko * C::ROWB + 16 * at(d4 >> 3) + 2 * (d4 & 7));
       bytes = perm((h >> 4) & 0x0F0Fu, h & 0x0F0Fu, 0x05010400u);
     }
     const h2 sbp = __builtin_bit_cast(h2, sbt[kb + ko]);
@@ -352,11 +383,11 @@ __device__ __forceinline__ void stage_k(const uint8_t* raw, _Float16* klds, int 
   const uint8_t* kr = raw + key * C::ROWB;
   uint32_t w[4];  // the half's 16 codes
   if constexpr (BITS == 8) {
-    const u4 a = *(const u4*)(kr + 16 * ((2 * q + H) ^ C::swz(key)));
+    const u4 a = *(const u4*)(kr + 16 * C::pos(key, 2 * q + H));
 #pragma unroll
     for (int i = 0; i < 4; ++i) w[i] = a[i];
   } else {
-    const u2 a = *(const u2*)(kr + 16 * (q ^ C::swz(key)) + 8 * H);
+    const u2 a = *(const u2*)(kr + 16 * C::pos(key, q) + 8 * H);
     w[0] = a[0];
     w[1] = a[1];
   }
@@ -1024,7 +1055,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   // ---- output. A lane holds 8-byte pieces of one row; stored directly, each store instruction
   // would write 8 bytes into each of 32 rows. Each wave instead stages its 32 rows in LDS (the
   // rings are free once every wave is past this barrier) and stores whole rows: 16 bytes a lane, so
-  // an instruction writes 4 (D = 128) or 8 (D = 64) complete rows.
+  // an instruction writes 4 (D = 128) or 8 (D = 64) complete rows (D = 96: 5 1/3).
   // (after a split merge l_tot and oacc are in true units; else the V operands' 2^-ev returns here)
   const float inv = l_tot > 0.0f ? (1.0f / l_tot) * (p.nsplit > 1 ? 1.0f : vback) : 0.0f;
   constexpr int OP = D + 8;                 // fp16 per staged row: rows shift by 4 banks
@@ -1050,11 +1081,11 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   const int roff_lo = (int)(uint32_t)roff, roff_hi = (int)(roff >> 32);
   __builtin_amdgcn_wave_barrier();  // the wave's LDS writes are issued before its reads (LDS keeps a wave's order)
   constexpr int CPR = D / 8;   // 16-byte chunks per row
-  constexpr int RPI = 64 / CPR;  // rows per store instruction
-  const int cc = lane % CPR;
 #pragma unroll
-  for (int it = 0; it < 32 / RPI; ++it) {
-    const int r = it * RPI + lane / CPR;
+  for (int it = 0; it < CPR / 2; ++it) {
+    constexpr bool whole = 64 % CPR == 0;  // a store instruction covers whole rows
+    const int r = whole ? it * (64 / CPR) + lane / CPR : (64 * it + lane) / CPR;
+    const int cc = whole ? lane % CPR : (64 * it + lane) % CPR;
     const u4 v = *(const u4*)(stage + r * OP + 8 * cc);
     const int64_t ro = (int64_t)(((uint64_t)(uint32_t)__shfl(roff_hi, r) << 32) | (uint32_t)__shfl(roff_lo, r));
     if (fr0 + wave * 32 + r < p.nrows) {
@@ -1097,6 +1128,12 @@ static PreLayout prefill_layout(const PrePlan& pl, int D) {
   return l;
 }
 
+// The plan with as many splits as `bytes` of workspace hold (at 64 and 128 dims always all of them).
+static PrePlan fit_plan(PrePlan pl, int D, size_t bytes) {
+  while (pl.nsplit > 1 && prefill_layout(pl, D).total > bytes) --pl.nsplit;
+  return pl;
+}
+
 size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window, int) {
   const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window);
   if (pl.nsplit == 1) return 256;
@@ -1110,7 +1147,8 @@ static hipError_t launch_prefill_t(const PreParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The quantized instantiation for (dtype, D in {64, 128}, bits in {4, 8}, G in {32, 64, 128}, G <= D).
+// The quantized instantiation for (dtype, D in {64, 128}, bits in {4, 8}, G in {32, 64, 128}, G <= D) or
+// (dtype, D = 96, bits, G = 32).
 template <bool PAGED>
 static hipError_t launch_prefill_quant(const PreParams& p, int dtype, int D, int bits, int G, hipStream_t stream) {
   auto by_g = [&](auto t, auto d, auto b) -> hipError_t {
@@ -1118,12 +1156,17 @@ static hipError_t launch_prefill_quant(const PreParams& p, int dtype, int D, int
     constexpr int DD = decltype(d)::value;
     constexpr int BB = decltype(b)::value;
     if (G == 32) return launch_prefill_t<TT, BB, PAGED, 32, DD>(p, stream);
-    if constexpr (DD >= 128) {
-      if (G == 128) return launch_prefill_t<TT, BB, PAGED, 128, DD>(p, stream);
+    if constexpr (DD == 96) {
+      return hipErrorInvalidValue;
+    } else {
+      if constexpr (DD >= 128) {
+        if (G == 128) return launch_prefill_t<TT, BB, PAGED, 128, DD>(p, stream);
+      }
+      return launch_prefill_t<TT, BB, PAGED, 64, DD>(p, stream);
     }
-    return launch_prefill_t<TT, BB, PAGED, 64, DD>(p, stream);
   };
   auto by_d = [&](auto t, auto b) -> hipError_t {
+    if (D == 96) return by_g(t, std::integral_constant<int, 96>{}, b);
     return D == 64 ? by_g(t, std::integral_constant<int, 64>{}, b) : by_g(t, std::integral_constant<int, 128>{}, b);
   };
   auto by_b = [&](auto t) -> hipError_t {
@@ -1167,8 +1210,9 @@ static PreParams prefill_params(const kvq_rows* q, const int32_t* seq_lens, cons
 
 hipError_t launch_prefill(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const int32_t* seq_lens,
                           const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype,
-                          float scale, int causal, int window, void* workspace, hipStream_t stream) {
-  const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window);
+                          float scale, int causal, int window, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream) {
+  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window), D, workspace_bytes);
   PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
   p.kc = (const uint8_t*)k->codes;
   p.vc = (const uint8_t*)v->codes;
@@ -1196,8 +1240,8 @@ hipError_t launch_prefill(const kvq_rows* q, const kvq_qtensor* k, const kvq_qte
 hipError_t launch_prefill_paged(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, int num_pages,
                                 const int32_t* table, int64_t table_stride, const int32_t* seq_lens, const kvq_rows* out,
                                 int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype, float scale,
-                                int causal, int window, void* workspace, hipStream_t stream) {
-  const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window);
+                                int causal, int window, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window), D, workspace_bytes);
   PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
   p.kc = (const uint8_t*)k->codes;
   p.vc = (const uint8_t*)v->codes;

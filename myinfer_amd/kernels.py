@@ -311,8 +311,11 @@ def decode_rows_per_pass(D: int, group_size: int = 64) -> int:
 def _auto_kernel(rep_rows: int, D: int, group_size: int) -> str:
     """Decode while a KV head's query rows fit at most two decode passes over its keys (one pass for
     group 64, where 8 rows fit one pass), the prefill kernel otherwise (head dims 64, 128 and 256 have
-    one; the others run the decode kernel at every length). At head_dim 256 the unquantized entry
-    points run the head_dim-256 kernel for every query length."""
+    one; the others run the decode kernel at every length, but for quantized caches of 96 dims (groups
+    of 32), which have a prefill kernel past 64 rows). At head_dim 256 the unquantized
+    entry points run the head_dim-256 kernel for every query length."""
+    if D == 96 and group_size == 32:
+        return "decode" if rep_rows <= 64 else "prefill"
     if D not in NATIVE_HEAD_DIMS:
         return "decode"
     return "decode" if rep_rows <= max(decode_rows_per_pass(D, group_size), 8) else "prefill"
@@ -452,11 +455,11 @@ def prepare_attention(queries: torch.Tensor, keys, values, scale: float, *, caus
         args = (ctypes.byref(qr), ctypes.byref(kq), ctypes.byref(vq), sl_ptr, ctypes.byref(orr), B, Hq, Hkv, L, D, S,
                 *tail)
     else:
-        # the caches' range words: registered with their buffers, else (one-shot prefill calls)
+        # the caches' range words: registered with their buffers, else (one-shot bf16 prefill calls)
         # computed from the scales and biases on the device; decode applies scales in fp32 and
-        # reads none
+        # reads none, and an fp16 cache's values always fit the operands
         kw, vw = range_word(keys[0]), range_word(values[0])
-        if kernel == "prefill" and _one_shot:
+        if kernel == "prefill" and _one_shot and queries.dtype == torch.bfloat16:
             kw = range_exponent(keys, bits) if kw is None else kw
             vw = range_exponent(values, bits) if vw is None else vw
         kq, vq = _lib.qtensor(*keys, range_exp=kw), _lib.qtensor(*values, range_exp=vw)
