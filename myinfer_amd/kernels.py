@@ -308,17 +308,39 @@ def decode_rows_per_pass(D: int, group_size: int = 64) -> int:
     return 16 * group_size // kernel_dim(D)
 
 
-def _auto_kernel(rep_rows: int, D: int, group_size: int) -> str:
-    """Decode while a KV head's query rows fit at most two decode passes over its keys (one pass for
-    group 64, where 8 rows fit one pass), the prefill kernel otherwise (head dims 64, 128 and 256 have
-    one; the others run the decode kernel at every length, but for quantized caches of 96 dims (groups
-    of 32), which have a prefill kernel past 64 rows). At head_dim 256 the unquantized
-    entry points run the head_dim-256 kernel for every query length."""
-    if D == 96 and group_size == 32:
+def _auto_kernel(rep_rows: int, D: int, group_size: int, *, dense: bool, units: int, keys: int) -> str:
+    """Decode or prefill for `units` (sequence, KV head) pairs of `rep_rows` query rows over `keys` keys.
+
+    Decode while a KV head's rows fit at most two decode passes over its keys (one pass for group 64,
+    where 8 rows fit one pass). Past that, over quantized caches and below the rows of one prefill
+    workgroup (256, or 128 at 256 dims), the kernel that is faster: a decode call's time grows with its
+    passes (about 25 us per 2^20 passes x units x keys at 128 dims), a prefill kernel's is that of the
+    whole row block and of merging the splits that a few such blocks are cut into. Measured at 128 dims,
+    8 bits, decode against prefill in us:
+      4 units, 8192 keys: 13.7 / 45.5 at 40 rows, 32.5 / 47 at 192;
+      16 units, 32768 keys: 57 / 81 at 32 rows, 105 / 83 at 48; 32 units, 32768 keys: 113 / 133 at 32;
+      prompts, where causality halves the prefill kernel's work: 32 units 7.8 / 11.6 at 128 tokens (512
+      row blocks, the last that run at once), 15.1 / 16.8 at 200, 25.5 / 18.2 at 330;
+    at 256 dims (4 rows a pass) 22 / 24 at 16 rows, 28 / 24 at 24 (8 units, 8192 keys), 57 / 59 at 16
+    rows of 32768 keys. Unquantized caches keep to one pass.
+
+    Head dims 64, 128 and 256 have prefill kernels; the others run the decode kernel at every length,
+    but for quantized caches of 96 dims (groups of 32), which have one past 64 rows. At head_dim 256 the
+    unquantized entry points run the head_dim-256 kernel for every query length."""
+    if D == 96 and not dense:
         return "decode" if rep_rows <= 64 else "prefill"
     if D not in NATIVE_HEAD_DIMS:
         return "decode"
-    return "decode" if rep_rows <= max(decode_rows_per_pass(D, group_size), 8) else "prefill"
+    per = decode_rows_per_pass(D, group_size)
+    if rep_rows <= max(per, 8):
+        return "decode"
+    if dense:
+        return "prefill"
+    passes, work = -(-rep_rows // per), units * keys
+    block, free, limit = (128, 3, 5 << 15) if D == 256 else (256, 4, 400_000)
+    if rep_rows < block and units * passes <= 512 and (passes - free) * work <= limit:
+        return "decode"
+    return "prefill"
 
 
 class AttentionCall:
@@ -430,7 +452,8 @@ def prepare_attention(queries: torch.Tensor, keys, values, scale: float, *, caus
         sl_ptr = seq_lens.data_ptr()
     rep = Hq // Hkv
     if kernel == "auto":
-        kernel = _auto_kernel(rep * L, D, 64 if dense else group_size)
+        kernel = _auto_kernel(rep * L, D, 64 if dense else group_size, dense=dense, units=B * Hkv,
+                              keys=min(S, window + L) if window else S)
     if kernel not in ("decode", "prefill"):
         raise ValueError(f"kernel must be 'decode', 'prefill' or 'auto', got {kernel!r}")
     lib = _lib.lib()
@@ -476,8 +499,8 @@ def attention(queries: torch.Tensor, keys, values, scale: float, *, causal: bool
     """softmax(scale * q K^T + mask) V. queries [B, Hq, L, D]; keys/values either quantized triples
     (codes [B, Hkv, S, D*bits/32], scales/biases [B, Hkv, S, D/G]) or unquantized tensors
     [B, Hkv, S, D] in the queries' dtype; returns [B, Hq, L, D] (or fills `out`). kernel: "decode",
-    "prefill" or "auto" (decode while a KV head's query rows fit max(16*G/D, 8) columns, that is
-    at most two decode passes over its keys, prefill otherwise)."""
+    "prefill" or "auto" (decode while a KV head's query rows fit max(16*G/D, 8) columns, and past
+    that where its passes over the keys cost less than the prefill kernel's row blocks)."""
     return prepare_attention(queries, keys, values, scale, causal=causal, window=window, seq_lens=seq_lens,
                              group_size=group_size, bits=bits, out=out, kernel=kernel, _one_shot=True)()
 
@@ -666,7 +689,8 @@ def paged_attention(queries: torch.Tensor, k_pool: Triple, v_pool: Triple, block
         queries = _copy_for_one_shot(queries, "queries", True)
     out = _check_out(out, queries, dev)
     if kernel == "auto":
-        kernel = _auto_kernel((Hq // Hkv) * L, D, group_size)
+        kernel = _auto_kernel((Hq // Hkv) * L, D, group_size, dense=False, units=B * Hkv,
+                              keys=min(S, window + L) if window else S)
     lib = _lib.lib()
     ws_fn = lib.kvq_decode_workspace_size if kernel == "decode" else lib.kvq_prefill_workspace_size
     nbytes = ws_fn(B, Hq, Hkv, L, D, S, int(window))
