@@ -263,7 +263,7 @@ size_t kvq_prefill_workspace_size(int B, int Hq, int Hkv, int L, int D, int S, i
  * widths for any L (by the decode kernel up to 128 dims, by the head_dim-256 kernel past them; the
  * key rows must then be exactly D elements apart); rows 16-byte aligned with strides that are
  * multiples of 8 elements. At D = 256 both entry points run the head_dim-256 prefill kernel (any
- * L); the prefill entry point runs the same kernel at D = 64. At D = 128 the prefill entry point
+ * L). At D = 128 the prefill entry point
  * stores output rows 16 bytes at a time, so out must be 16-byte aligned with strides in multiples
  * of 8 elements there too.
  */

@@ -393,12 +393,7 @@ size_t kvq_prefill_workspace_size(int B, int Hq, int Hkv, int L, int D, int S, i
   // the same size
   if (!native_dim(D)) return kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, window);
   if (D == 256) return kvq::wide_workspace_bytes(B, Hq, Hkv, L, D, S, window);
-  const size_t n = kvq::prefill_workspace_bytes(B, Hq, Hkv, L, D, S, window, 8);
-  if (D == 64) {  // the unquantized cache at head_dim 64 runs through wide.hip's kernel
-    const size_t x = kvq::wide_workspace_bytes(B, Hq, Hkv, L, D, S, window);
-    return x > n ? x : n;
-  }
-  return n;
+  return kvq::prefill_workspace_bytes(B, Hq, Hkv, L, D, S, window, 8);
 }
 
 // The prefill kernel loads two scale groups of a row at once when a row has several: scale and
@@ -586,11 +581,11 @@ int kvq_prefill_attn_dense(const kvq_rows* q, const kvq_rows* k, const kvq_rows*
     return hip_status(kvq::launch_decode_dense(q, k, v, seq_lens, out, B, Hq, Hkv, L, D, S, dtype, scale, causal, window,
                                                workspace, (hipStream_t)stream),
                       "prefill_attn_dense launch (the decode kernel, head_dim other than 64/128/256)");
-  if (D != 128)
+  if (D == 256)
     return hip_status(kvq::launch_wide_dense(q, k, v, seq_lens, out, B, Hq, Hkv, L, D, S, dtype, scale, causal, window,
                                              workspace, (hipStream_t)stream),
-                      "prefill_attn_dense launch (head_dim 64 / 256)");
-  if ((rc = check_rows(out, "out", D, true))) return rc;  // rows are stored 16 bytes at a time
+                      "prefill_attn_dense launch (head_dim 256)");
+  if (D == 128 && (rc = check_rows(out, "out", D, true))) return rc;  // rows are stored 16 bytes at a time
   return hip_status(kvq::launch_prefill_dense(q, k, v, seq_lens, out, B, Hq, Hkv, L, D, S, dtype, scale, causal, window,
                                               workspace, (hipStream_t)stream),
                     "prefill_attn_dense launch");

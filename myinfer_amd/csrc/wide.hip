@@ -1,8 +1,7 @@
 // Attention at head_dim 256: the reference's blocked attention over a quantized cache
 // (m5engine/attention.py:29-103) for models whose heads are 256 wide, and every call over an
 // unquantized cache of that width (the plain KVCache before quantized_kv_start and the sliding-window
-// RotatingKVCache, which the reference leaves to mlx-lm's SDPA, attention.py:106-112). The same
-// kernel at head_dim 64 serves prefill over unquantized caches of that width.
+// RotatingKVCache, which the reference leaves to mlx-lm's SDPA, attention.py:106-112).
 //
 //   out = softmax(scale * q K^T + mask) V,  K = sK * codesK + bK,  V = sV * codesV + bV
 //
@@ -53,7 +52,7 @@ template <int D, int BITS, int G>
 struct WideCfg {
   static constexpr bool DENSE = BITS == 16;
   static_assert(DENSE || ((BITS == 4 || BITS == 8) && (G == 64 || G == 128)), "4/8 bits, groups 64/128");
-  static_assert(D == 256 || (D == 64 && DENSE), "head_dim 256, or 64 over an unquantized cache");
+  static_assert(D == 256, "head_dim 256");
   static constexpr int NG = DENSE ? 1 : D / G;             // scale groups per row
   static constexpr int KSTEPS = D / 16;                    // QK MFMA k-steps
   static constexpr int NDB = D / 32;                       // PV MFMA column blocks
@@ -244,22 +243,17 @@ __device__ __forceinline__ void wide_stage_v(const uint8_t* raw, uint8_t* vop, i
   using C = WideCfg<D, BITS, G>;
   const int c = t >> 6, j = t & 63;
   const uint8_t* vraw = raw + C::TB;
-  // xp[e][q]: key e's dims 2q, 2q + 1 of the thread's VPT as a packed pair (one 16-bit value when
-  // VPT is 1)
-  uint32_t xp[8][(C::VPT + 1) / 2];
+  // xp[e][q]: key e's dims 2q, 2q + 1 of the thread's 4 as a packed pair
+  static_assert(C::VPT == 4, "head_dim 256");
+  uint32_t xp[8][2];
   if constexpr (C::DENSE) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      if constexpr (C::VPT == 4) {
-        const u2 v = *(const u2*)(vraw + w_slot_key(c, e) * C::ROWB + 8 * j);
-        xp[e][0] = v[0];
-        xp[e][1] = v[1];
-      } else {
-        xp[e][0] = *(const uint16_t*)(vraw + w_slot_key(c, e) * C::ROWB + 2 * j);
-      }
+      const u2 v = *(const u2*)(vraw + w_slot_key(c, e) * C::ROWB + 8 * j);
+      xp[e][0] = v[0];
+      xp[e][1] = v[1];
     }
   } else {
-    static_assert(C::VPT == 4, "quantized caches at head_dim 256");
     const int g = 4 * j / G;
     const uint8_t* cells = raw + 2 * C::TB + 2 * C::SBA + 4 * 32 * g;  // sV, then bV one array later
     const int kb0 = w_slot_key(c, 0);
@@ -286,11 +280,7 @@ __device__ __forceinline__ void wide_stage_v(const uint8_t* raw, uint8_t* vop, i
     u4 o;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
-      if constexpr (C::VPT == 1) {
-        o[a] = (xp[2 * a][0] & 0xffffu) | (xp[2 * a + 1][0] << 16);
-      } else {
-        o[a] = perm(xp[2 * a + 1][i >> 1], xp[2 * a][i >> 1], (i & 1) ? 0x07060302u : 0x05040100u);
-      }
+      o[a] = perm(xp[2 * a + 1][i >> 1], xp[2 * a][i >> 1], (i & 1) ? 0x07060302u : 0x05040100u);
     }
     // row d is stored at row d ^ ((d >> 4) & 1): the 8 consecutive lanes of a write (rows 4 apart)
     // then fill both 64-byte halves of a 128-byte bank window, 8 distinct 16-byte slots
@@ -827,8 +817,6 @@ hipError_t launch_wide_dense(const kvq_rows* q, const kvq_rows* k, const kvq_row
   p.vc_ss = v->stride_l * 2;
   p.dv = D;
   if (D > 128 && D < 256) D = 256;  // rows narrower than the kernel: read 256 wide at their own stride
-  if (D == 64)
-    return dtype == KVQ_DTYPE_BF16 ? launch_wide_t<BF16, 64, 16, 64>(p, stream) : launch_wide_t<F16, 64, 16, 64>(p, stream);
   if (D == 256)
     return dtype == KVQ_DTYPE_BF16 ? launch_wide_t<BF16, 256, 16, 64>(p, stream)
                                    : launch_wide_t<F16, 256, 16, 64>(p, stream);
