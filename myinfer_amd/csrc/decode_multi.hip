@@ -1,8 +1,8 @@
 // The decode kernel over several passes' query rows (speculative verification, short chunks and prompts:
 // some query positions times the heads of a GQA group). Each row block is a unit of its own whose
 // keys are read again, from L2 where the blocks run side by side: 64 rows of 4 KV heads over 8192
-// 8-bit keys take 13.9 us against 45.5 on the prefill kernel, whose workgroups compute 256 rows
-// whether they are there or not and merge 32 splits. (Several row groups computed in one workgroup
+// 8-bit keys take 14.4 us against 18.4 on the prefill kernel, whose workgroups compute 256 rows
+// whether they are there or not and take a launch to merge 32 splits. (Several row groups computed in one workgroup
 // over one reading of the keys measured the same or slower up to 40 rows: 16.6 against 17.5 us at
 // 40, 19.7 against 13.0 at 24; the groups' work is not hidden behind a 2-slot ring.)
 

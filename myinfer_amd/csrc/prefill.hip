@@ -7,20 +7,51 @@
 namespace kvq {
 
 struct PrePlan {
-  int rowblocks, nunits, nsplit;
+  int rowblocks, nunits, nsplit, chunk, longest_first;
 };
 
-static PrePlan prefill_plan(int B, int Hq, int Hkv, int L, int S, int window) {
+// Splits merged by the last of them to arrive; more take prefill_combine_kernel. Few splits are cheaper
+// in the kernel (the last 512-token chunk of 16384, 4 splits: 155.2 against 161.3 us for the layer
+// step), many in a launch of their own, whose loads run side by side: 64 rows of 4 KV heads over 8192
+// keys (32 splits) 45.5 -> 18.4 us, over 32768 (64 splits) 81.2 -> 28.0.
+constexpr int kPFusedMaxSplit = 4;
+
+static PrePlan prefill_plan(int B, int Hq, int Hkv, int L, int S, int window, int causal) {
   PrePlan pl;
-  const int nrows = (Hq / Hkv) * L;
+  const int rep = Hq / Hkv, nrows = rep * L;
   pl.rowblocks = (nrows + kPRows - 1) / kPRows;
   pl.nunits = B * Hkv * pl.rowblocks;
-  // keys a row block sees: the whole context, or about a window
+  // keys a row block sees: the whole context, or about a window; the first row block of a causal call
   const int span = window > 0 ? std::min(S, window + kPRows) : S;
-  const int tiles = (span + kPT - 1) / kPT;
+  const int first = causal && window == 0 ? std::min(S, S - L + (kPRows + rep - 1) / rep) : span;
+  const int tiles = (span + kPT - 1) / kPT, tiles0 = (first + kPT - 1) / kPT;
+  const int nbk = B * Hkv;
+  const bool unequal = 2 * tiles0 <= tiles;
   int ns = (kPTargetWgs + pl.nunits - 1) / pl.nunits;
+  if (unequal) {
+    // A causal prompt, whose first row blocks see few keys: the number of splits with the shortest
+    // estimate, in tiles (of about 2.2 us at 128 dims), of max(the longest workgroup, an even share of
+    // all work), a workgroup costing 4 tiles besides its own and 2 more where it takes part in a merge.
+    // 32 KV heads of 96 dims, 1999 tokens, 1 / 2 splits: 56 / 48 us; 4 KV heads of 8 query heads of
+    // 128 dims, 1000 tokens, 2 / 3 / 4 splits: 26.5 / 24.8 / 37.9 us.
+    const float avg = 0.5f * (tiles + tiles0);
+    float best = 0.0f;
+    for (int c = 1; c <= kPFusedMaxSplit; ++c) {
+      const int chunk = (tiles + c - 1) / c, cost = c > 1 ? 6 : 4;
+      const float total = pl.nunits * (avg + (avg / chunk + 0.5f) * cost);
+      const float est = std::max(total / kPTargetWgs, (float)(chunk + cost));
+      if (c == 1 || est < best) {
+        best = est;
+        ns = c;
+      }
+    }
+  }
   ns = std::min(ns, std::max(1, tiles / 4));  // at least about 4 tiles per split
   pl.nsplit = pl.nunits > kMaxCountedUnits ? 1 : std::max(1, std::min(ns, kMaxSplit));
+  pl.chunk = (tiles + pl.nsplit - 1) / pl.nsplit * kPT;
+  const bool dealt = nbk % kXcds == 0 ||
+                     (nbk < kXcds && kXcds % nbk == 0 && pl.rowblocks * pl.nsplit % (kXcds / nbk) == 0);
+  pl.longest_first = !unequal ? 0 : dealt ? 1 : 2;
   return pl;
 }
 
@@ -40,19 +71,25 @@ static PreLayout prefill_layout(const PrePlan& pl, int D) {
 // The plan with as many splits as `bytes` of workspace hold (at 64 and 128 dims always all of them).
 static PrePlan fit_plan(PrePlan pl, int D, size_t bytes) {
   while (pl.nsplit > 1 && prefill_layout(pl, D).total > bytes) --pl.nsplit;
-  return pl;
+  return pl;  // (fewer splits take longer chunks: split_keys)
 }
 
 size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window, int) {
-  const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window);
-  if (pl.nsplit == 1) return 256;
-  return prefill_layout(pl, D).total;
+  size_t n = 256;
+  for (int causal : {0, 1}) {
+    const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window, causal);
+    if (pl.nsplit > 1) n = std::max(n, prefill_layout(pl, D).total);
+  }
+  return n;
 }
 
 template <typename T, int BITS, bool PAGED = false, int G = 64, int D = 128>
 static hipError_t launch_prefill_t(const PreParams& p, hipStream_t stream) {
   hipLaunchKernelGGL((prefill_attn_kernel<T, BITS, PAGED, G, D>), dim3(p.nunits * p.nsplit), dim3(kPW * 64), 0, stream,
                      p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || p.nsplit == 1 || p.fused) return e;
+  hipLaunchKernelGGL((prefill_combine_kernel<T, D>), dim3(p.nunits * kPW * (D / 16)), dim3(kPW * 64), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -109,6 +146,9 @@ static PreParams prefill_params(const kvq_rows* q, const int32_t* seq_lens, cons
   p.nrows = p.rep * L;
   p.rowblocks = pl.rowblocks;
   p.nsplit = pl.nsplit;
+  p.chunk = pl.chunk;
+  p.longest_first = pl.longest_first;
+  p.fused = pl.nsplit <= kPFusedMaxSplit;
   p.nunits = pl.nunits;
   p.xcd_remap = ((int64_t)pl.nunits * pl.nsplit) % kXcds == 0;
   p.scale_log2 = scale * 1.4426950408889634f;
@@ -121,7 +161,7 @@ hipError_t launch_prefill(const kvq_rows* q, const kvq_qtensor* k, const kvq_qte
                           const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype,
                           float scale, int causal, int window, void* workspace, size_t workspace_bytes,
                           hipStream_t stream) {
-  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window), D, workspace_bytes);
+  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window, causal), D, workspace_bytes);
   PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
   p.kc = (const uint8_t*)k->codes;
   p.vc = (const uint8_t*)v->codes;
@@ -150,7 +190,7 @@ hipError_t launch_prefill_paged(const kvq_rows* q, const kvq_qtensor* k, const k
                                 const int32_t* table, int64_t table_stride, const int32_t* seq_lens, const kvq_rows* out,
                                 int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype, float scale,
                                 int causal, int window, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window), D, workspace_bytes);
+  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window, causal), D, workspace_bytes);
   PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
   p.kc = (const uint8_t*)k->codes;
   p.vc = (const uint8_t*)v->codes;
@@ -181,7 +221,7 @@ hipError_t launch_prefill_paged(const kvq_rows* q, const kvq_qtensor* k, const k
 hipError_t launch_prefill_dense(const kvq_rows* q, const kvq_rows* k, const kvq_rows* v, const int32_t* seq_lens,
                                 const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int dtype,
                                 float scale, int causal, int window, void* workspace, hipStream_t stream) {
-  const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window);
+  const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window, causal);
   PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
   p.kc = (const uint8_t*)k->data;
   p.vc = (const uint8_t*)v->data;

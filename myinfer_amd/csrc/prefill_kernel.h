@@ -151,7 +151,11 @@ struct PreParams {
   float* part_ml;
   unsigned* counters;  // arrivals per unit, zero between launches
   int xcd_remap;       // 1: the grid is a multiple of the XCD count (see the numbering in the kernel)
+  int longest_first;   // row blocks of unequal length, numbered from the longest down: 1 over all (sequence,
+                       // KV head) pairs of an XCD, 2 within each pair
   int Hq, Hkv, L, S, rep, nrows, rowblocks, nsplit, nunits;
+  int chunk;           // keys per split (a multiple of 64); see split_keys
+  int fused;           // 1: the last split of a row block merges; 0: prefill_combine_kernel does
   float scale_log2;
   int causal, window;
   // paged cache (PAGED kernels): rows of sequence b live in 64-row pages, page table[b][r / 64];
@@ -165,6 +169,23 @@ struct PreParams {
   const int32_t* v_rexp;
   int out8;  // 1: output rows are only 8-byte aligned (unquantized head_dim 64)
 };
+
+// The keys the rows [fr0, frl] of a row block see, in whole tiles ([lo, hi), lo rounded down to a
+// tile), and the splits they are cut into: `chunk` keys each, so that workgroups of long and short
+// row blocks (a causal prompt's last and first) are about as long, the short ones taking fewer.
+struct KeySplit {
+  int lo, hi, chunk, nsplit;
+};
+__device__ __forceinline__ KeySplit split_keys(const PreParams& p, int S_b, int fr0, int frl) {
+  const int pos_min = S_b - p.L + fr0 / p.rep, pos_max = S_b - p.L + frl / p.rep;
+  KeySplit k;
+  k.hi = p.causal ? min(S_b, pos_max + 1) : S_b;
+  k.lo = (p.window > 0 ? max(0, pos_min - p.window + 1) : 0) & ~(kPT - 1);
+  const int span = max(k.hi - k.lo, 0);
+  k.chunk = max(p.chunk, ((span + p.nsplit - 1) / p.nsplit + kPT - 1) / kPT * kPT);
+  k.nsplit = max((span + k.chunk - 1) / k.chunk, 1);
+  return k;
+}
 
 // V^T slot of key `kk` (0..63) inside a tile: the 16 keys of PV k-step j = kk / 16 are stored so
 // that slots 16j + 8h + i hold the keys the score layout gives lane half h at i.
@@ -475,14 +496,35 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   // Workgroup numbering: the row blocks of one (sequence, KV head, split) share every K/V tile, so
   // they are consecutive, and consecutive workgroups are placed on one XCD (the hardware hands
   // workgroups to the 8 XCDs in turn): each tile is fetched into one L2 rather than eight.
-  int wg = blockIdx.x;
-  if (p.xcd_remap) {
-    const int per_xcd = (int)(gridDim.x / kXcds);
-    wg = (wg % kXcds) * per_xcd + wg / kXcds;
+  int rb, split, bk;  // bk = b * Hkv + kvh
+  if (p.longest_first == 1) {
+    // a causal prompt, whose last row blocks see many times the keys of its first: every XCD takes its
+    // share of the (sequence, KV head) pairs (or a pair's row blocks are dealt to several XCDs) and
+    // runs the row blocks of all of them from the longest down, so that short ones fill the end
+    const int x = blockIdx.x % kXcds, i = blockIdx.x / kXcds, nbk = (int)gridDim.x / (p.rowblocks * p.nsplit);
+    int rank;
+    if (nbk >= kXcds) {
+      const int mine = nbk / kXcds;
+      bk = x * mine + i % mine;
+      rank = i / mine;
+    } else {
+      const int per = kXcds / nbk;
+      bk = x / per;
+      rank = i * per + x % per;
+    }
+    rb = p.rowblocks - 1 - rank / p.nsplit;
+    split = rank % p.nsplit;
+  } else {
+    int wg = blockIdx.x;
+    if (p.xcd_remap) {
+      const int per_xcd = (int)(gridDim.x / kXcds);
+      wg = (wg % kXcds) * per_xcd + wg / kXcds;
+    }
+    rb = wg % p.rowblocks;
+    if (p.longest_first) rb = p.rowblocks - 1 - rb;
+    split = (wg / p.rowblocks) % p.nsplit;
+    bk = wg / (p.rowblocks * p.nsplit);
   }
-  const int rb = wg % p.rowblocks;
-  const int split = (wg / p.rowblocks) % p.nsplit;
-  const int bk = wg / (p.rowblocks * p.nsplit);  // b * Hkv + kvh
   const int b = bk / p.Hkv, kvh = bk % p.Hkv;
   const int unit = bk * p.rowblocks + rb;
   const int S_b = p.seq_lens ? min(max(load_uniform_i32(p.seq_lens, b), 0), p.S) : p.S;
@@ -490,18 +532,15 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   // ---- the workgroup's rows, their positions, and the key range they see
   const int fr0 = rb * kPRows;
   const int frl = min(fr0 + kPRows, p.nrows) - 1;
+  const KeySplit ks = split_keys(p, S_b, fr0, frl);
+  if (split >= ks.nsplit) return;
+  const int nsplit = ks.nsplit;
   const int pos_min = S_b - p.L + fr0 / p.rep, pos_max = S_b - p.L + frl / p.rep;
-  const int hi_wg = p.causal ? min(S_b, pos_max + 1) : S_b;
-  const int lo_wg = p.window > 0 ? max(0, pos_min - p.window + 1) : 0;
   // keys every row of the workgroup sees: tiles inside need no mask
   const int hi_all = p.causal ? min(S_b, pos_min + 1) : S_b;
   const int lo_all = p.window > 0 ? max(0, pos_max - p.window + 1) : 0;
-  // splits cover [lo_wg rounded down to a tile, hi_wg) in whole tiles (tile starts stay 64-aligned)
-  const int lo_al = lo_wg & ~(kPT - 1);
-  const int span = max(hi_wg - lo_al, 0);
-  const int chunk = ((span + p.nsplit - 1) / p.nsplit + kPT - 1) / kPT * kPT;
-  const int k_begin = lo_al + split * chunk;
-  const int k_end = min(k_begin + chunk, hi_wg);
+  const int k_begin = ks.lo + split * ks.chunk;  // tile starts stay 64-aligned
+  const int k_end = min(k_begin + ks.chunk, ks.hi);
   const int ntile = k_end > k_begin ? (k_end - k_begin + kPT - 1) / kPT : 0;
 
   // ---- this lane's query row (MFMA column qc of this wave)
@@ -956,7 +995,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
 
   // ---- epilogue: this lane holds O^T[d][row] for d = 32db + 8(i/4) + 4hh + i%4
   float l_tot = add_xor32(l_run);
-  if (p.nsplit > 1) {
+  if (nsplit > 1) {
     // Key split: publish this split's partials, count the arrival, and let the unit's last split to
     // arrive merge them into its own registers.
     //  * A partial row is o / l in fp16, times 2^-e with e chosen per row so every stored value is
@@ -1004,18 +1043,19 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
 #pragma unroll
     for (int u = 0; u < QW; ++u) store_agent_b128(ro, lo + u * 1024 + split * split_o, __builtin_bit_cast(f4, own[u]));
     if (hh == 0) store_agent_b128(rm, row_ml + split * (kPRows * 16), f4{m_run, l_tot, own_sc, 0.0f});
+    if (!p.fused) return;
     // The stores are acknowledged (written through to the device's coherence point) before the
     // arrival is counted, so the last arrival sees every split's partials.
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (tid == 0) *s_arrived = __hip_atomic_fetch_add(&p.counters[unit], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (*s_arrived != (unsigned)(p.nsplit - 1)) return;
+    if (*s_arrived != (unsigned)(nsplit - 1)) return;
     if (tid == 0) __hip_atomic_store(&p.counters[unit], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
     // M = max over the splits that saw a key; weights 2^(m_s - M)
     float M = l_tot > 0.0f ? m_run : -INFINITY;
-    for (int s2 = 0; s2 < p.nsplit; ++s2) {
+    for (int s2 = 0; s2 < nsplit; ++s2) {
       if (s2 == split) continue;
       const f4 rec = load_agent_b128(rm, row_ml, s2 * (kPRows * 16));
       if (rec[1] > 0.0f) M = fmaxf(M, rec[0]);
@@ -1025,7 +1065,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
 #pragma unroll
     for (int db = 0; db < NDB; ++db) macc[db] = f16v{};
     float l_acc = 0.0f;
-    for (int s2 = 0; s2 < p.nsplit; ++s2) {
+    for (int s2 = 0; s2 < nsplit; ++s2) {
       f4 rec;
       u4 po[QW];
       if (s2 == split) {
@@ -1065,7 +1105,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   // rings are free once every wave is past this barrier) and stores whole rows: 16 bytes a lane, so
   // an instruction writes 4 (D = 128) or 8 (D = 64) complete rows (D = 96: 5 1/3).
   // (after a split merge l_tot and oacc are in true units; else the V operands' 2^-ev returns here)
-  const float inv = l_tot > 0.0f ? (1.0f / l_tot) * (p.nsplit > 1 ? 1.0f : vback) : 0.0f;
+  const float inv = l_tot > 0.0f ? (1.0f / l_tot) * (nsplit > 1 ? 1.0f : vback) : 0.0f;
   constexpr int OP = D + 8;                 // fp16 per staged row: rows shift by 4 banks
   constexpr int WSB = 32 * OP * 2;          // staging bytes per wave
   constexpr int NRW = kRawSlots * RC::SLOT / WSB;           // waves staged in the raw ring
@@ -1104,6 +1144,94 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
         *(u4*)(p.out + ro + 8 * cc) = v;  // the host checks 16-byte aligned rows and strides
       }
     }
+  }
+}
+
+// The split merge as a launch of its own, for row blocks cut into many splits: in the kernel above the
+// last split loads the others one after another (about 0.9 us each at 128 dims). A workgroup takes one
+// 16-byte word u of the packed rows of one wave (32 rows) of a row block; its 8 waves take the splits
+// in turn, four in flight each, and wave 0 sums the eight partial merges. Row blocks that were not
+// split have been written already.
+template <typename T, int D>
+__global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) {
+  constexpr int QW = D / 16;
+  __shared__ float s_m[kPW][64], s_l[kPW][64];
+  __shared__ __align__(16) float s_o[kPW][64][8];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int u = blockIdx.x % QW, w = (blockIdx.x / QW) % kPW, unit = blockIdx.x / (QW * kPW);
+  const int rb = unit % p.rowblocks, bk = unit / p.rowblocks;
+  const int b = bk / p.Hkv, kvh = bk % p.Hkv;
+  const int S_b = p.seq_lens ? min(max(load_uniform_i32(p.seq_lens, b), 0), p.S) : p.S;
+  const int fr0 = rb * kPRows, frl = min(fr0 + kPRows, p.nrows) - 1;
+  const KeySplit ks = split_keys(p, S_b, fr0, frl);
+  if (ks.nsplit == 1 || fr0 + 32 * w >= p.nrows) return;
+  const uint8_t* po = (const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * (kPRows * 2 * D) + (w * QW + u) * 1024 + 16 * lane;
+  const f4* rec = (const f4*)(p.part_ml + (int64_t)unit * p.nsplit * (kPRows * 4)) + 32 * w + (lane & 31);
+  constexpr int CH = 4;
+  float M = -INFINITY, l = 0.0f, acc[8] = {};
+  for (int s0 = wave; s0 < ks.nsplit; s0 += kPW * CH) {
+    f4 r[CH];
+    u4 v[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int s = min(s0 + kPW * i, ks.nsplit - 1);  // past the last split it is re-read, and not counted
+      r[i] = rec[s * kPRows];
+      v[i] = *(const u4*)(po + (int64_t)s * (kPRows * 2 * D));
+    }
+    float Mn = M;
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+      if (s0 + kPW * i < ks.nsplit && r[i][1] > 0.0f) Mn = fmaxf(Mn, r[i][0]);
+    const float corr = M == Mn ? 1.0f : exp2_fast(M - Mn);
+    l *= corr;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= corr;
+    M = Mn;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      if (s0 + kPW * i >= ks.nsplit) continue;
+      // a row that saw no key in the split counts 0, but for NaN (a poisoned row block)
+      const float wl = r[i][1] > 0.0f ? exp2_fast(r[i][0] - M) * r[i][1] : 0.0f;
+      l += wl;
+      const float F = wl * r[i][2];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t x = v[i][e >> 1];
+        acc[e] = fmaf(F, (float)__builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? x >> 16 : x & 0xffffu)), acc[e]);
+      }
+    }
+  }
+  s_m[wave][lane] = M;
+  s_l[wave][lane] = l;
+#pragma unroll
+  for (int e = 0; e < 8; e += 4) *(f4*)&s_o[wave][lane][e] = f4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
+  __syncthreads();
+  const int row = fr0 + 32 * w + (lane & 31);
+  if (wave != 0 || row >= p.nrows) return;
+  M = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < kPW; ++k) M = fmaxf(M, s_m[k][lane]);
+  l = 0.0f;
+  f4 o[2] = {};
+#pragma unroll
+  for (int k = 0; k < kPW; ++k) {
+    const float f = s_m[k][lane] == -INFINITY ? (M == -INFINITY ? 1.0f : 0.0f) : exp2_fast(s_m[k][lane] - M);
+    l += f * s_l[k][lane];
+    o[0] += f * *(const f4*)&s_o[k][lane][0];
+    o[1] += f * *(const f4*)&s_o[k][lane][4];
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  // word u packs value groups 2u and 2u + 1; group 4 db + c holds dims 32 db + 8 c + 4 hh .. + 3
+  uint16_t* dst = p.out + (int64_t)b * p.o_sb + (int64_t)(kvh * p.rep + row % p.rep) * p.o_sh +
+                  (int64_t)(row / p.rep) * p.o_sl + 4 * (lane >> 5);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int g = 2 * u + h;
+    u2 x;
+    x[0] = (uint32_t)from_float(o[h][0] * inv, T{}) | ((uint32_t)from_float(o[h][1] * inv, T{}) << 16);
+    x[1] = (uint32_t)from_float(o[h][2] * inv, T{}) | ((uint32_t)from_float(o[h][3] * inv, T{}) << 16);
+    *(u2*)(dst + 32 * (g >> 2) + 8 * (g & 3)) = x;
   }
 }
 

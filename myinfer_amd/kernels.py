@@ -317,8 +317,8 @@ def _auto_kernel(rep_rows: int, D: int, group_size: int, *, dense: bool, units: 
     passes (about 25 us per 2^20 passes x units x keys at 128 dims), a prefill kernel's is that of the
     whole row block and of merging the splits that a few such blocks are cut into. Measured at 128 dims,
     8 bits, decode against prefill in us:
-      4 units, 8192 keys: 13.7 / 45.5 at 40 rows, 32.5 / 47 at 192;
-      16 units, 32768 keys: 57 / 81 at 32 rows, 105 / 83 at 48; 32 units, 32768 keys: 113 / 133 at 32;
+      4 units, 8192 keys: 14.4 / 18.4 at 64 rows, 20.1 / 19.9 at 128; 2048 keys: 13.4 / 18.2 at 192;
+      16 units, 32768 keys: 57 / 72 at 32 rows, 105 / 72 at 48; 32 units, 32768 keys: 110 / 131 at 32;
       prompts, where causality halves the prefill kernel's work: 32 units 7.8 / 11.6 at 128 tokens (512
       row blocks, the last that run at once), 15.1 / 16.8 at 200, 25.5 / 18.2 at 330;
     at 256 dims (4 rows a pass) 22 / 24 at 16 rows, 28 / 24 at 24 (8 units, 8192 keys), 57 / 59 at 16
@@ -337,7 +337,7 @@ def _auto_kernel(rep_rows: int, D: int, group_size: int, *, dense: bool, units: 
     if dense:
         return "prefill"
     passes, work = -(-rep_rows // per), units * keys
-    block, free, limit = (128, 3, 5 << 15) if D == 256 else (256, 4, 400_000)
+    block, free, limit = (128, 3, 5 << 15) if D == 256 else (256, 4, 330_000)
     if rep_rows < block and units * passes <= 512 and (passes - free) * work <= limit:
         return "decode"
     return "prefill"
