@@ -211,8 +211,10 @@ typedef struct kvq_mask {
  * masks that are not causal, sliding-window or right-padding masks, per-head masks and additive
  * masks. Replaces: m5engine/attention.py:55-56 and :76-80 (the array-mask branches of the
  * blocked loop) and the mask handling of the L == 1 hand-off at :42-45. The decode kernel reads
- * the mask beside each 32-key tile; rows beyond one pass take more passes over the keys, so long
- * prompts under such masks run at the decode kernel's rate. Same requirements and workspace
+ * the mask beside each 32-key tile; rows beyond one pass take more passes over the keys. Calls of many
+ * rows and keys run on the prefill kernel instead (head_dim 64, 96 or 128, a boolean mask, output rows
+ * it can store, and for a bf16 cache range words): a first launch finds the tiles no row sees, which
+ * are skipped, and those all rows see, which are computed without the mask. Same requirements and workspace
  * (kvq_decode_workspace_size with window 0) as kvq_decode_attn.
  */
 int kvq_decode_attn_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v,
@@ -221,7 +223,8 @@ int kvq_decode_attn_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qt
                            void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * The same over an unquantized cache (kvq_decode_attn_dense's arguments and head dims).
+ * The same over an unquantized cache (kvq_decode_attn_dense's arguments and head dims; the prefill kernel
+ * takes boolean and additive masks there, at head_dim 64 and 128).
  * Replaces the mask handling of mx.fast.scaled_dot_product_attention for array masks.
  */
 int kvq_decode_attn_dense_masked(const kvq_rows* q, const kvq_rows* k, const kvq_rows* v,

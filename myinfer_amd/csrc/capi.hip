@@ -348,6 +348,10 @@ size_t kvq_decode_workspace_size(int B, int Hq, int Hkv, int L, int D, int S, in
       const size_t x = kvq::decode_workspace_bytes(B, Hq, Hkv, L, D, S, window, bits, G);
       n = x > n ? x : n;
     }
+  if (window == 0 && Hq % Hkv == 0) {  // calls under a general mask may run on the prefill kernel
+    const size_t x = kvq::prefill_masked_bytes(B, Hq, Hkv, L, D, S);
+    n = x > n ? x : n;
+  }
   if (Dk == 256) {  // unquantized rows past 128 dims run through the head_dim-256 kernel
     const size_t x = kvq::wide_workspace_bytes(B, Hq, Hkv, L, Dk, S, window);
     n = x > n ? x : n;
@@ -538,6 +542,25 @@ static int check_mask(const kvq_mask* m) {
   return KVQ_OK;
 }
 
+// Whether a call under a general mask runs on the prefill kernel: enough query rows per KV head, a head
+// dim it has, rows it can store, a cache whose values its operands hold (a bf16 cache needs its range
+// words), and over a quantized cache a boolean mask (the tile loop's scalar registers hold no more than
+// that reading). The others stay on the decode kernel.
+static bool masked_on_prefill(const kvq_qtensor* k, const kvq_qtensor* v, const kvq_rows* out, int B, int Hq, int Hkv, int L,
+                              int D, int S, int group_size, int dtype, const kvq_mask* mask, size_t ws_bytes) {
+  if (!kvq::prefill_masked_rows(B, Hq, Hkv, L, D, S)) return false;
+  const bool rows16 = aligned(out->data, 16) && !((out->stride_b | out->stride_h | out->stride_l) % 8);
+  if (!k) {
+    if (D != 64 && (D != 128 || !rows16)) return false;
+  } else {
+    if (mask->kind != KVQ_MASK_BOOL) return false;
+    if ((D != 64 && D != 96 && D != 128) || !rows16) return false;
+    if (D != 96 && check_prefill_sb(k, v, D, group_size)) return false;
+    if (dtype == KVQ_DTYPE_BF16 && (!k->range_exp || !v->range_exp)) return false;
+  }
+  return kvq::prefill_masked_fits(B, Hq, Hkv, L, D, S, mask, ws_bytes);
+}
+
 int kvq_decode_attn_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const kvq_rows* out, int B,
                            int Hq, int Hkv, int L, int D, int S, int bits, int group_size, int dtype, float scale,
                            const kvq_mask* mask, void* workspace, size_t workspace_bytes, void* stream) {
@@ -545,6 +568,11 @@ int kvq_decode_attn_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qt
   int rc = check_attn(q, k, v, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale, 0,
                       kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0), workspace, workspace_bytes);
   if (rc || (rc = check_mask(mask))) return rc;
+  const size_t ws = kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0);
+  if (masked_on_prefill(k, v, out, B, Hq, Hkv, L, D, S, group_size, dtype, mask, ws))
+    return hip_status(kvq::launch_prefill_masked(q, k, v, nullptr, nullptr, out, B, Hq, Hkv, L, D, S, bits, group_size,
+                                                 dtype, scale, mask, workspace, ws, (hipStream_t)stream),
+                      "decode_attn_masked launch (the prefill kernel)");
   return hip_status(kvq::launch_decode(q, k, v, nullptr, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale, 0, 0,
                                        workspace, (hipStream_t)stream, mask),
                     "decode_attn_masked launch");
@@ -561,6 +589,11 @@ int kvq_decode_attn_dense_masked(const kvq_rows* q, const kvq_rows* k, const kvq
     return hip_status(kvq::launch_wide_dense(q, k, v, nullptr, out, B, Hq, Hkv, L, D, S, dtype, scale, 0, 0, workspace,
                                              (hipStream_t)stream, mask),
                       "decode_attn_dense_masked launch (the head_dim-256 kernel)");
+  const size_t ws = kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0);
+  if (masked_on_prefill(nullptr, nullptr, out, B, Hq, Hkv, L, D, S, 64, dtype, mask, ws))
+    return hip_status(kvq::launch_prefill_masked(q, nullptr, nullptr, k, v, out, B, Hq, Hkv, L, D, S, 16, 64, dtype, scale,
+                                                 mask, workspace, ws, (hipStream_t)stream),
+                      "decode_attn_dense_masked launch (the prefill kernel)");
   return hip_status(kvq::launch_decode_dense(q, k, v, nullptr, out, B, Hq, Hkv, L, D, S, dtype, scale, 0, 0, workspace,
                                              (hipStream_t)stream, mask),
                     "decode_attn_dense_masked launch");

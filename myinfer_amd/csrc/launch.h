@@ -51,6 +51,17 @@ hipError_t launch_prefill_paged(const kvq_rows* q, const kvq_qtensor* k, const k
                                 const int32_t* table, int64_t table_stride, const int32_t* seq_lens, const kvq_rows* out,
                                 int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype, float scale,
                                 int causal, int window, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// Under a general mask: bits 16 over kd / vd (head_dim 64 or 128), else over k / v (64, 96 or 128);
+// workspace_bytes as for launch_prefill.
+// prefill_masked_rows: whether the prefill kernel is the faster one for such a call; prefill_masked_bytes:
+// the workspace it would have then (0 else).
+bool prefill_masked_rows(int B, int Hq, int Hkv, int L, int D, int S);
+size_t prefill_masked_bytes(int B, int Hq, int Hkv, int L, int D, int S);
+bool prefill_masked_fits(int B, int Hq, int Hkv, int L, int D, int S, const kvq_mask* mask, size_t workspace_bytes);
+hipError_t launch_prefill_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const kvq_rows* kd,
+                                 const kvq_rows* vd, const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S,
+                                 int bits, int G, int dtype, float scale, const kvq_mask* mask, void* workspace,
+                                 size_t workspace_bytes, hipStream_t stream);
 // wide.hip: head_dim 256 over quantized (4/8 bits, groups 64/128) and unquantized caches, any query length
 size_t wide_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window);
 hipError_t launch_wide(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const int32_t* seq_lens,

@@ -168,7 +168,40 @@ struct PreParams {
   const int32_t* k_rexp;
   const int32_t* v_rexp;
   int out8;  // 1: output rows are only 8-byte aligned (unquantized head_dim 64)
+  // general mask (kvq_mask; MASKED kernels), over the reference's grouped score layout, and what
+  // mask_classes_kernel found in it: per row block (and KV head, if the mask has one: w_kv units of
+  // row blocks apart) 2 words per 64 tiles, [any][mixed], bit i of word w being tile 64 w + i
+  const void* mask;
+  int mask_kind;
+  int64_t m_sb, m_skv, m_srep, m_sl;
+  const uint64_t* words;
+  int nwords;  // words per bitmap
+  int w_kv;    // 1: the bitmaps have a KV head axis
 };
+
+// The tiles of a row block that hold a visible key, under a general mask, and how the splits share
+// them: `chunk` tiles of that list each.
+struct MaskSplit {
+  const uint64_t* any;    // [nwords], then the mixed bitmap
+  int n, chunk, nsplit;
+};
+__device__ __forceinline__ uint64_t load_uniform_u64(const uint64_t* p, int i) {
+  return ((const __attribute__((address_space(4))) uint64_t*)p)[i];
+}
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) |
+         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32);
+}
+__device__ __forceinline__ MaskSplit split_masked(const PreParams& p, int b, int kvh, int rb) {
+  MaskSplit m;
+  m.any = p.words + (int64_t)((p.w_kv ? b * p.Hkv + kvh : b) * p.rowblocks + rb) * (2 * p.nwords);
+  m.n = 0;
+  for (int w = 0; w < p.nwords; ++w) m.n += __builtin_popcountll(load_uniform_u64(m.any, w));
+  m.n = __builtin_amdgcn_readfirstlane(m.n);  // (wave-uniform, as everything the tile walk is made of)
+  m.chunk = max(p.chunk / kPT, (m.n + p.nsplit - 1) / p.nsplit);
+  m.nsplit = max((m.n + m.chunk - 1) / m.chunk, 1);
+  return m;
+}
 
 // The keys the rows [fr0, frl] of a row block see, in whole tiles ([lo, hi), lo rounded down to a
 // tile), and the splits they are cut into: `chunk` keys each, so that workgroups of long and short
@@ -471,8 +504,11 @@ __device__ __forceinline__ void stage_v_raw(const uint8_t* raw, _Float16* vlds, 
   *(u4*)&vlds[(2 * d2 + 1) * kVS + 8 * c8] = hi;
 }
 
-template <typename T, int BITS, bool PAGED = false, int G = 64, int D = 128>
+// MASKED: 0, or under a general mask: 1 boolean, 2 additive. The tile loop then walks the list of tiles
+// with a visible key, and reads the mask beside those that are not visible as a whole.
+template <typename T, int BITS, bool PAGED = false, int G = 64, int D = 128, int MASKED = 0>
 __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) {
+  static_assert(!(PAGED && MASKED), "general masks: contiguous caches");
   using RC = RawCfg<BITS, G, D>;
   constexpr bool DENSE = RC::DENSE;  // unquantized cache: K operands are read from the raw ring
   constexpr int KS = kKS<D>;
@@ -532,16 +568,61 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   // ---- the workgroup's rows, their positions, and the key range they see
   const int fr0 = rb * kPRows;
   const int frl = min(fr0 + kPRows, p.nrows) - 1;
-  const KeySplit ks = split_keys(p, S_b, fr0, frl);
-  if (split >= ks.nsplit) return;
-  const int nsplit = ks.nsplit;
+  KeySplit ks;
+  MaskSplit ms;
+  if constexpr (MASKED) {
+    ms = split_masked(p, b, kvh, rb);
+  } else {
+    ks = split_keys(p, S_b, fr0, frl);
+  }
+  const int nsplit = MASKED ? ms.nsplit : ks.nsplit;
+  if (split >= nsplit) return;
   const int pos_min = S_b - p.L + fr0 / p.rep, pos_max = S_b - p.L + frl / p.rep;
   // keys every row of the workgroup sees: tiles inside need no mask
   const int hi_all = p.causal ? min(S_b, pos_min + 1) : S_b;
   const int lo_all = p.window > 0 ? max(0, pos_max - p.window + 1) : 0;
-  const int k_begin = ks.lo + split * ks.chunk;  // tile starts stay 64-aligned
-  const int k_end = min(k_begin + ks.chunk, ks.hi);
-  const int ntile = k_end > k_begin ? (k_end - k_begin + kPT - 1) / kPT : 0;
+  int k_begin = 0, ntile;  // tile starts stay 64-aligned
+  if constexpr (MASKED) {
+    ntile = __builtin_amdgcn_readfirstlane(max(min(ms.chunk, ms.n - split * ms.chunk), 0));
+  } else {
+    k_begin = ks.lo + split * ks.chunk;
+    const int k_end = min(k_begin + ks.chunk, ks.hi);
+    ntile = k_end > k_begin ? (k_end - k_begin + kPT - 1) / kPT : 0;
+  }
+  // under a mask: the walk over the listed tiles (the word in hand, its index, tiles left to hand out),
+  // and the tiles handed out but not yet computed, in order (bit 31: mixed)
+  uint64_t wk_any = 0, wk_mixed = 0;
+  int wk_w = -1, wk_left = ntile, wk_last = 0;
+  int tq[4] = {0, 0, 0, 0};
+  auto next_tile = [&]() -> int {
+    if (wk_left > 0) {
+      while (wk_any == 0) {
+        ++wk_w;
+        wk_any = uniform64(load_uniform_u64(ms.any, wk_w));
+        wk_mixed = uniform64(load_uniform_u64(ms.any, p.nwords + wk_w));
+      }
+      const int i = __builtin_ctzll(wk_any);
+      wk_any &= wk_any - 1;
+      --wk_left;
+      wk_last = (64 * wk_w + i) | ((int)((wk_mixed >> i) & 1) << 31);
+    }
+    return __builtin_amdgcn_readfirstlane(wk_last);  // past the last tile it is handed out again
+  };
+  if constexpr (MASKED) {
+    if (ntile > 0) {
+      // skip the tiles of the splits before this one
+      int skip = split * ms.chunk;
+      for (;;) {
+        ++wk_w;
+        wk_any = uniform64(load_uniform_u64(ms.any, wk_w));
+        const int c = __builtin_popcountll(wk_any);
+        if (skip < c) break;
+        skip -= c;
+      }
+      for (; skip > 0; --skip) wk_any &= wk_any - 1;
+      wk_mixed = uniform64(load_uniform_u64(ms.any, p.nwords + wk_w));
+    }
+  }
 
   // ---- this lane's query row (MFMA column qc of this wave)
   const int fr = fr0 + wave * 32 + qc;
@@ -593,7 +674,12 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   };
   int pg_next = PAGED ? page_of(k_begin) : 0;
   auto issue_raw = [&](int i) {
-    const int k0 = k_begin + kPT * min(i, last);
+    int k0 = k_begin + kPT * min(i, last);
+    if constexpr (MASKED) {  // tiles are issued in order, each once: the queue holds those not computed yet
+      const int e = next_tile();
+      tq[min(i, DENSE ? 2 : 3)] = e;
+      k0 = kPT * (e & 0x7fffffff);
+    }
     const uint32_t slot = raw_lds + (i % kRawSlots) * RC::SLOT;
     if constexpr (PAGED) {
       const int pg = pg_next;
@@ -661,6 +747,71 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
 #pragma unroll
       for (int i = 0; i < 4; ++i) qop[j][i] = pack_f16x2(qv[j][2 * i] * qmul, qv[j][2 * i + 1] * qmul);
   }
+  // ---- under a mask the scores are brought to log2 units as they are masked (an additive mask is added
+  // there), so the softmax that follows applies no scale of its own
+  const float sinv = MASKED ? 1.0f : inv2;
+  const uint8_t* mrow = nullptr;
+  if constexpr (MASKED) {
+    const int el = MASKED == 1 ? 1 : p.mask_kind == KVQ_MASK_F32 ? 4 : 2;
+    mrow = (const uint8_t*)p.mask +
+           el * ((int64_t)b * p.m_sb + (int64_t)kvh * p.m_skv + (int64_t)(head - kvh * p.rep) * p.m_srep + (int64_t)lq * p.m_sl);
+  }
+  // the 16 scores of the 32-key block from k (this lane's keys k + 8 c + 4 hh + e, its mask row mrow)
+  auto general_mask = [&](f16v& acc, int k, bool mixed) {
+    if (!mixed) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] *= inv2;
+      return;
+    }
+    const bool whole = k + 32 <= p.S;  // else the row of the mask ends inside the block
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int t = k + 8 * c + 4 * hh;
+      if constexpr (MASKED == 1) {
+        uint32_t m = 0;
+        if (whole) {
+          __builtin_memcpy(&m, mrow + t, 4);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (t + e < p.S) m |= (uint32_t)mrow[t + e] << (8 * e);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[4 * c + e] = (m >> (8 * e)) & 0xffu ? acc[4 * c + e] * inv2 : -INFINITY;
+      } else {
+        float a[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        if (p.mask_kind == KVQ_MASK_F32) {
+          if (whole) {
+            __builtin_memcpy(a, mrow + 4 * (int64_t)t, 16);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (t + e < p.S) a[e] = ((const float*)mrow)[t + e];
+          }
+        } else {
+          uint16_t r[4] = {0, 0, 0, 0};
+          if (whole) {
+            __builtin_memcpy(r, mrow + 2 * (int64_t)t, 8);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (t + e < p.S) r[e] = ((const uint16_t*)mrow)[t + e];
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (whole || t + e < p.S) a[e] = p.mask_kind == KVQ_MASK_BF16 ? to_float(r[e], BF16{}) : to_float(r[e], F16{});
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[4 * c + e] = fmaf(acc[4 * c + e], inv2, a[e] * 1.4426950408889634f);
+        if (!whole) {  // keys past the end stay hidden whatever their score was
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (t + e >= p.S) acc[4 * c + e] = -INFINITY;
+        }
+      }
+    }
+  };
   // MFMA operand type: bf16 for an unquantized bf16 cache, else fp16
   using OT = typename std::conditional<DENSE && T::id == KVQ_DTYPE_BF16, BF16, F16>::type;
 
@@ -675,6 +826,13 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
     // window edge need a mask (a branch the whole workgroup takes or skips); there, each element's
     // offset c = 32kb + 8(i/4) + i%4 is a constant compared with the lane's bounds
     auto mask_tile = [&](f16v (&acc)[2], int k0) {
+      if constexpr (MASKED) {
+        general_mask(acc[0], kPT * (tq[0] & 0x7fffffff), tq[0] < 0);
+        general_mask(acc[1], kPT * (tq[0] & 0x7fffffff) + 32, tq[0] < 0);
+        tq[0] = tq[1];
+        tq[1] = tq[2];
+        return;
+      }
       const bool need_mask = !(k0 >= lo_all && k0 + kPT <= hi_all);
       if (__builtin_expect(need_mask, 0)) {
         const int lo = lo_r - k0 - 4 * hh, hi = hi_r - k0 - 4 * hh;
@@ -703,7 +861,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) tm = fmaxf(tm, acc[kb][i]);
-      tm = max_xor32(tm) * inv2;
+      tm = max_xor32(tm) * sinv;
       if (__builtin_amdgcn_ballot_w64(tm > m_run + kPSlack) != 0) {
         const float m_new = tm > m_run + kPSlack ? fmaxf(m_run, tm) : m_run;
         const float corr = m_new == m_run ? 1.0f : exp2_fast(m_run - m_new);
@@ -725,8 +883,8 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
       for (int j = 0; j < 4; ++j) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float p0 = exp2_fast(fmaf(acc[j >> 1][8 * (j & 1) + 2 * e], inv2, nm));
-          const float p1 = exp2_fast(fmaf(acc[j >> 1][8 * (j & 1) + 2 * e + 1], inv2, nm));
+          const float p0 = exp2_fast(fmaf(acc[j >> 1][8 * (j & 1) + 2 * e], sinv, nm));
+          const float p1 = exp2_fast(fmaf(acc[j >> 1][8 * (j & 1) + 2 * e + 1], sinv, nm));
           pop[j][e] = pack2(p0, p1, OT{});
           lsum[e & 1] = add_pair(pop[j][e], lsum[e & 1], OT{});
         }
@@ -821,7 +979,11 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
     using J0 = std::integral_constant<int, 0>;
     using JE = std::integral_constant<int, KSTEPS>;
     // the block's keys [k, k + 32): mask (only on a causal diagonal or window edge), row maximum
-    auto mask_blk = [&](f16v& acc, int k) {
+    auto mask_blk = [&](f16v& acc, int k, int entry) {
+      if constexpr (MASKED) {
+        general_mask(acc, k, entry < 0);
+        return;
+      }
       if (__builtin_expect(!(k >= lo_all && k + 32 <= hi_all), 0)) {
         const int lo = lo_r - k - 4 * hh, hi = hi_r - k - 4 * hh;
 #pragma unroll
@@ -835,7 +997,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
       float tm = -INFINITY;
 #pragma unroll
       for (int i = 0; i < 16; ++i) tm = fmaxf(tm, acc[i]);
-      return max_xor32(tm) * inv2;
+      return max_xor32(tm) * sinv;
     };
     auto rescale = [&](float tm) {
       if (__builtin_amdgcn_ballot_w64(tm > m_run + kPSlack) != 0) {
@@ -857,8 +1019,8 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float p0 = exp2_fast(fmaf(acc[8 * j + 2 * e], inv2, nm));
-          const float p1 = exp2_fast(fmaf(acc[8 * j + 2 * e + 1], inv2, nm));
+          const float p0 = exp2_fast(fmaf(acc[8 * j + 2 * e], sinv, nm));
+          const float p1 = exp2_fast(fmaf(acc[8 * j + 2 * e + 1], sinv, nm));
           pop[j][e] = pack2(p0, p1, OT{});
           lsum[e & 1] = add_pair(pop[j][e], lsum[e & 1], OT{});
         }
@@ -897,14 +1059,20 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
         stage_v_table<T, BITS, G, D>(raw2, sb_tab[wave & 3], tid, range_bad, vmul);
         __builtin_amdgcn_wave_barrier();
       }
-      const int k0 = k_begin + kPT * t;
+      const int entry = MASKED ? tq[0] : 0;
+      const int k0 = MASKED ? kPT * (entry & 0x7fffffff) : k_begin + kPT * t;
+      if constexpr (MASKED) {
+        tq[0] = tq[1];
+        tq[1] = tq[2];
+        tq[2] = tq[3];
+      }
       const _Float16* vl = vl_lane + v_t;
       u4 ring[4];
       u4 pop[2];
       // half 0: softmax of block 0 beside S(block 1) = K(t) rows 32-63 Q^T
       {
         const _Float16* kl = kl_lane + k_t + 32 * KS;
-        mask_blk(sX, k0);
+        mask_blk(sX, k0, entry);
         const float tm = max_blk(sX);
         rescale(tm);
         qk_ring(ring, kl);
@@ -920,7 +1088,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
       // half 1: softmax of block 1 beside S(block 0 of tile t + 1) = K(t + 1) rows 0-31 Q^T
       {
         const _Float16* kl = kl_lane + k_t1;
-        mask_blk(sY, k0 + 32);
+        mask_blk(sY, k0 + 32, entry);
         const float tm = max_blk(sY);
         rescale(tm);
         if constexpr (QKN) {
@@ -1152,7 +1320,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
 // 16-byte word u of the packed rows of one wave (32 rows) of a row block; its 8 waves take the splits
 // in turn, four in flight each, and wave 0 sums the eight partial merges. Row blocks that were not
 // split have been written already.
-template <typename T, int D>
+template <typename T, int D, bool MASKED = false>
 __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) {
   constexpr int QW = D / 16;
   __shared__ float s_m[kPW][64], s_l[kPW][64];
@@ -1164,7 +1332,14 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
   const int b = bk / p.Hkv, kvh = bk % p.Hkv;
   const int S_b = p.seq_lens ? min(max(load_uniform_i32(p.seq_lens, b), 0), p.S) : p.S;
   const int fr0 = rb * kPRows, frl = min(fr0 + kPRows, p.nrows) - 1;
-  const KeySplit ks = split_keys(p, S_b, fr0, frl);
+  struct {
+    int nsplit;
+  } ks;
+  if constexpr (MASKED) {
+    ks.nsplit = split_masked(p, b, kvh, rb).nsplit;
+  } else {
+    ks.nsplit = split_keys(p, S_b, fr0, frl).nsplit;
+  }
   if (ks.nsplit == 1 || fr0 + 32 * w >= p.nrows) return;
   const uint8_t* po = (const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * (kPRows * 2 * D) + (w * QW + u) * 1024 + 16 * lane;
   const f4* rec = (const f4*)(p.part_ml + (int64_t)unit * p.nsplit * (kPRows * 4)) + 32 * w + (lane & 31);
@@ -1234,5 +1409,8 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
     *(u2*)(dst + 32 * (g >> 2) + 8 * (g & 3)) = x;
   }
 }
+
+// prefill_masked.hip: the MASKED launches and the kernel that classes the mask's tiles.
+hipError_t launch_prefill_masked_t(const PreParams& p, int B, int dtype, int D, int bits, int G, hipStream_t stream);
 
 }  // namespace kvq

@@ -601,7 +601,8 @@ def masked_attention(queries: torch.Tensor, keys, values, scale: float, mask: to
                                               B, Hq, Hkv, L, D, S, _lib.dtype_code(queries.dtype), *tail)
         _lib.check(rc, "kvq_decode_attn_dense_masked")
     else:
-        kq, vq = _lib.qtensor(*keys), _lib.qtensor(*values)
+        kq = _lib.qtensor(*keys, range_exp=range_word(keys[0]))
+        vq = _lib.qtensor(*values, range_exp=range_word(values[0]))
         rc = lib.kvq_decode_attn_masked(ctypes.byref(qr), ctypes.byref(kq), ctypes.byref(vq), ctypes.byref(orr), B, Hq,
                                         Hkv, L, D, S, int(bits), int(group_size), _lib.dtype_code(queries.dtype), *tail)
         _lib.check(rc, "kvq_decode_attn_masked")
