@@ -3,7 +3,8 @@
 The HIP sources under ``csrc/`` are compiled for gfx950 with hipcc and linked against the HIP
 runtime that PyTorch ships (``torch/lib/libamdhip64.so``), so the library, torch's allocator and
 torch's streams all live in one HIP runtime instance. The library is written next to this file
-(``libkvq.so``) so it travels with the source tree.
+(``libkvq.so``) so it travels with the source tree, and so is the host path over torch tensors
+(``_kvqhost.so``: csrc/host, g++ against torch's headers).
 
 Usage: ``python -m myinfer_amd._build`` or ``myinfer_amd._build.build()``.
 """
@@ -15,12 +16,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OBJ = PKG / "_build"
 LIB = PKG / "libkvq.so"
+HOST = PKG / "_kvqhost.so"  # the host path over torch tensors (csrc/host)
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -86,16 +89,23 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
         raise RuntimeError(f"no HIP sources in {CSRC}")
     objs = [OBJ / (s.stem + ".o") for s in sources]
     host_objs = [OBJ / (s.stem + ".host.o") for s in host_sources]
-    jobs = jobs or min(len(sources) + len(host_sources), max(1, os.cpu_count() or 1), 8)
+    tlib = _torch_lib_dir()
+    host_tmp = HOST.with_suffix(".so.tmp")
+    tinc = tlib.parent / "include"
+    host_cmd = ["g++", *HOST_FLAGS, "-shared", "-w", f"-I{tinc}", f"-I{tinc}/torch/csrc/api/include",
+                f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host" / "host.cpp"), "-o", str(host_tmp), f"-L{tlib}",
+                "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{tlib}"]
+    jobs = jobs or min(len(sources) + len(host_sources) + 1, max(1, os.cpu_count() or 1), 8)
     with cf.ThreadPoolExecutor(jobs) as ex:
         futs = [ex.submit(_run, [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(s.name, []), "-c", str(s), "-o", str(o)], verbose)
                 for s, o in zip(sources, objs)]
         futs += [ex.submit(_run, ["g++", *HOST_FLAGS, "-c", str(s), "-o", str(o)], verbose)
                  for s, o in zip(host_sources, host_objs)]
+        futs.append(ex.submit(_run, host_cmd, verbose))
         for f in futs:
             f.result()
+    os.replace(host_tmp, HOST)
     objs += host_objs
-    tlib = _torch_lib_dir()
     tmp = LIB.with_suffix(".so.tmp")
     link = [
         "g++",

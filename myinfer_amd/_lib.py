@@ -252,4 +252,33 @@ def qtensor(codes: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
+class AppendState(ctypes.Structure):
+    """The destination of an AppendCall as the native host path reads it (csrc/host/host.cpp)."""
+
+    _fields_ = [("fn", c_void_p), ("kq", c_void_p), ("vq", c_void_p), ("rope", c_void_p), ("B", c_int64), ("H", c_int64),
+                ("rows", c_int64), ("code_words", c_int64), ("groups", c_int64), ("bits", ctypes.c_int32),
+                ("group", ctypes.c_int32), ("code", ctypes.c_int32), ("device", ctypes.c_int32), ("stream", c_void_p)]
+
+
+_host = None
+
+
+def host():
+    """The native host path (``_kvqhost.so``), bound to the library's entry points. Raises if it is missing."""
+    global _host
+    if _host is None:
+        handle = lib()
+        try:
+            from . import _kvqhost
+        except ImportError as e:
+            raise ImportError(f"_kvqhost.so does not load ({e}): build it with `python -m myinfer_amd._build`") from e
+        with _lock:
+            if _host is None:
+                _kvqhost.bind(*(ctypes.cast(fn, c_void_p).value for fn in (
+                    handle.kvq_decode_attn, handle.kvq_prefill_attn, handle.kvq_decode_workspace_size,
+                    handle.kvq_prefill_workspace_size)))
+                _host = _kvqhost
+    return _host

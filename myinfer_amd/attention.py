@@ -165,6 +165,11 @@ def blocked_quantized_sdpa(queries: torch.Tensor, q_keys, q_values, scale: float
     Query head h reads KV head h // (Hq / Hkv) (:47-53). Returns [B, Hq, L, D] in the queries'
     dtype. Rows that see no key return 0, as the reference's blocked path does.
     """
+    if mask is None or type(mask) is str:
+        out = kernels.layer_attention(queries, q_keys, q_values, scale, causal=mask is not None or bool(window),
+                                      window=window, seq_lens=seq_lens, group_size=group_size, bits=bits)
+        if out is not None:
+            return out
     B, n_q_heads, L, D = queries.shape
     S = q_keys[0].shape[-2]
     try:

@@ -21,7 +21,7 @@ from typing import List, Optional, Tuple
 
 import torch
 
-from . import kernels
+from . import _lib, kernels
 
 STEP = 256
 
@@ -311,7 +311,7 @@ class QuantizedKVCache:
         if self.keys is None or prev + L > self.keys[0].shape[2]:
             self._resize(keys, values, L)
         # the append's descriptors are built once per buffer set, RoPE and stream
-        key = (id(self.keys[0]), id(self.values[0]), rope, torch.cuda.current_stream(keys.device).cuda_stream)
+        key = (id(self.keys[0]), id(self.values[0]), rope, _lib.stream_ptr(keys.device))
         if getattr(self, "_append_key", None) != key:
             self._append = kernels.prepare_append(self.keys, self.values, group_size=self.group_size,
                                                   bits=self.bits, rope=rope)
@@ -323,6 +323,9 @@ class QuantizedKVCache:
     def fetch(self):
         """The (codes, scales, biases) views of the first `offset` rows, for K and for V."""
         o = self.offset
+        both = _lib.host().views(self.keys, self.values, o)
+        if both is not None:
+            return both
         return tuple(x[..., :o, :] for x in self.keys), tuple(x[..., :o, :] for x in self.values)
 
     @property

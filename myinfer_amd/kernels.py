@@ -216,9 +216,19 @@ class AppendCall:
         lib = _lib.lib()
         self._fn = lib.kvq_rope_quantize_append if rope is not None else lib.kvq_quantize_append
         self._stream = _lib.stream_ptr(self._dev)
+        self._host = _lib.host().append
+        self._state = _lib.AppendState(
+            ctypes.cast(self._fn, ctypes.c_void_p).value, ctypes.addressof(self._kq),
+            None if self._vq is None else ctypes.addressof(self._vq),
+            None if self._rp is None else ctypes.addressof(self._rp), *self._lead, self._rows, *self._widths, self._bits,
+            self._group, self._code, self._dev.index, self._stream)
+        self._state_ptr = ctypes.addressof(self._state)
 
     def __call__(self, k: torch.Tensor, v: Optional[torch.Tensor], row_offset: int,
                  rope_offset: Optional[int] = None) -> None:
+        # the native host path; anything it does not take is checked, served or refused below
+        if self._host(self._state_ptr, k, v, row_offset, row_offset if rope_offset is None else rope_offset):
+            return
         if k.dtype != self._dtype or k.device != self._dev or k.dim() != 4 or k.stride(-1) != 1:
             raise ValueError("rows must match the prepared dtype and device, as [B, H, L, D] with D contiguous")
         B, H, L, D = k.shape
@@ -491,6 +501,40 @@ def prepare_attention(queries: torch.Tensor, keys, values, scale: float, *, caus
         keep_words = (kw, vw)
     keep = (queries, keys, values, seq_lens, ws, qr, orr, kq, vq) + (() if dense else keep_words)
     return AttentionCall(fn, args, keep, kernel, out, symbol)
+
+
+def layer_attention(queries: torch.Tensor, keys, values, scale: float, *, causal: bool, window: int = 0,
+                    seq_lens: Optional[torch.Tensor] = None, group_size: int = 64,
+                    bits: int = 8) -> Optional[torch.Tensor]:
+    """``attention`` over a quantized cache through the native host path, for the calls a model's layers
+    make (the same checks, kernels and results); None for any other form, which ``attention`` then serves
+    or refuses."""
+    if not (torch.is_tensor(queries) and queries.is_cuda and queries.dim() == 4 and type(keys) is tuple and
+            type(values) is tuple and len(keys) == 3):
+        return None
+    B, Hq, L, D = queries.shape
+    if D not in NATIVE_HEAD_DIMS and D != 96:
+        return None
+    Hkv, S = keys[0].shape[1:3] if keys[0].dim() == 4 else (0, 0)
+    if not Hkv or Hq % Hkv or group_size not in (32, 64, 128) or type(window) is not int:
+        return None
+    prefill = _auto_kernel(Hq // Hkv * L, D, group_size, dense=False, units=B * Hkv,
+                           keys=min(S, window + L) if window else S) == "prefill"
+    kw = vw = None
+    if prefill and queries.dtype == torch.bfloat16:  # the range words, which only these kernels read
+        kw, vw = range_word(keys[0]), range_word(values[0])
+        if kw is None or vw is None:
+            return None
+    dev = queries.device.index
+    stream = torch._C._cuda_getCurrentRawStream(dev)
+    ws = _workspaces.get((dev, stream))
+    args = (queries, keys, values, float(scale), int(causal), window, seq_lens, group_size, bits, int(prefill),
+            0 if kw is None else kw.data_ptr(), 0 if vw is None else vw.data_ptr())
+    call = _lib.host().attention
+    out = call(*args, ws, stream)
+    if type(out) is int:  # the bytes of workspace it needs
+        out = call(*args, _workspace(queries.device, stream, out), stream)
+    return out
 
 
 def attention(queries: torch.Tensor, keys, values, scale: float, *, causal: bool = False,

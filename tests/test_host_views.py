@@ -1,0 +1,29 @@
+"""The native path's cache views on the CPU: the slices Python would take, and what it hands back."""
+
+import torch
+
+from myinfer_amd import _lib
+
+
+def test_views_are_slices():
+    h = _lib.host()
+    tr = tuple(torch.arange(2 * 3 * 8 * w).view(2, 3, 8, w) for w in (4, 2, 2))
+    for n in (0, 1, 5, 8):
+        both = h.views(tr, tr, n)
+        assert type(both) is tuple and len(both) == 2
+        for got in both:
+            for a, b in zip(got, tr):
+                s = b[..., :n, :]
+                assert torch.equal(a, s) and a.stride() == s.stride() and a.storage_offset() == s.storage_offset()
+    both = h.views(tr, tr, 3)
+    both[0][0].fill_(-1)  # a view, not a copy
+    assert bool((tr[0][..., :3, :] == -1).all())
+
+
+def test_handed_back():
+    h = _lib.host()
+    tr = tuple(torch.zeros(1, 1, 4, 2) for _ in range(3))
+    assert h.views(list(tr), tr, 2) is None and h.views(tr, tr[:2], 2) is None
+    assert h.views(tr, tr, 5) is None and h.views(tr, tr, -1) is None
+    assert h.attention(tr[0], tr, tr, 0.1, 0, 0, None, 64, 8, 0, 0, 0, None, 0) is None  # CPU tensors
+    assert h.append(0, tr[0], tr[0], 0, 0) is None
