@@ -14,7 +14,10 @@
 //
 // Thread mapping: one thread per 32 (large launches) or 8 consecutive elements, 16 bytes a load, all
 // loads in flight at once; the threads of a group are neighbouring lanes and reduce min/max with
-// DPP lane permutes. Grid.y selects the K or the V job of one launch.
+// DPP lane permutes. Grid.y selects the K or the V job of one launch. A large append is bound by its
+// bytes and by instruction issue about equally: with codes of 16-byte aligned rows stored 16 bytes at a
+// time and bytes made by v_cvt_pk_u8_f32 (clamp, conversion and insertion in one), 2048 rows of 4
+// sequences of 16 heads of 128 dims, K and V in 8 bits (103 MB), went from 27.5 to 24.2 us (4.3 TB/s).
 //
 // RoPE (kvq_rope_quantize_append): the K job rotates its rows before quantizing, the way mlx-lm's
 // attention layers rotate keys before the cache update and the reference's native kernel fuses
@@ -40,11 +43,48 @@ struct RopeArgs {
   float freq[kMaxRopePairs];
 };
 
-// cos and sin of the angle of pair `pair` at position `pos`
-__device__ __forceinline__ void rope_cs(const RopeArgs& r, int64_t pos, int pair, float& c, float& s) {
+// The angle of pair `pair` at position `pos`.
+__device__ __forceinline__ float rope_angle(const RopeArgs& r, int64_t pos, int pair) {
 #pragma clang fp contract(off)
-  const float ang = ((float)pos * r.scale) * r.freq[pair];
-  sincosf(ang, &s, &c);
+  return ((float)pos * r.scale) * r.freq[pair];
+}
+
+// cos and sin of N angles, the arithmetic that bounds a rotating append (its bytes take a third of its time).
+// Below 2^26 an angle is k pi/2 + t, |t| <= pi/4, reduced in double (one FMA: off by k 2^-53 at most, below
+// 5e-9 here), where the library's reduction of a large angle is a long integer sequence; then the Taylor
+// series of sin and cos about 0 to t^9 and t^10 (remainders 1.8e-9 and 1.2e-10). Against sincosf, the append
+// of 2048 rows of 8 heads of 256 dims went from 20.3 to 16.4 us (8 elements a thread). The low part of t
+// that the float drops is added back to the sine.
+template <int N>
+__device__ __forceinline__ void rope_cs(const float (&ang)[N], float (&c)[N], float (&s)[N]) {
+#pragma clang fp contract(off)
+  bool far = false;
+#pragma unroll
+  for (int e = 0; e < N; ++e) far |= !(fabsf(ang[e]) < 0x1p26f);  // (and NaN)
+  if (__builtin_expect(far, 0)) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) sincosf(ang[e], &s[e], &c[e]);
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    const double k = __builtin_rint((double)ang[e] * 0.63661977236758134308);
+    const double td = __builtin_fma(-k, 1.57079632679489661923, (double)ang[e]);
+    const float t = (float)td, tl = (float)(td - (double)t), z = t * t;
+    float sn = __builtin_fmaf(z, 2.7557319e-6f, -1.9841270e-4f);
+    sn = __builtin_fmaf(z, sn, 8.3333333e-3f);
+    sn = __builtin_fmaf(z, sn, -1.6666667e-1f);
+    sn = t + __builtin_fmaf(t * z, sn, tl);
+    float cn = __builtin_fmaf(z, -2.7557319e-7f, 2.4801587e-5f);
+    cn = __builtin_fmaf(z, cn, -1.3888889e-3f);
+    cn = __builtin_fmaf(z, cn, 4.1666667e-2f);
+    cn = __builtin_fmaf(z, cn, -0.5f);
+    cn = __builtin_fmaf(z, cn, 1.0f);
+    const int quadrant = (int)k;
+    const float a = quadrant & 1 ? cn : sn, b = quadrant & 1 ? sn : cn;
+    s[e] = quadrant & 2 ? -a : a;
+    c[e] = (quadrant + 1) & 2 ? -b : b;
+  }
 }
 
 static RopeArgs make_rope_args(const kvq_rope_params* p) {
@@ -64,23 +104,25 @@ __device__ __forceinline__ void rope8(const RopeArgs& r, int64_t pos, int d0, fl
 #pragma clang fp contract(off)
   if (d0 >= r.dims) return;
   if (r.traditional) {
+    float ang[4], c[4], sn[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ang[i] = rope_angle(r, pos, d0 / 2 + i);
+    rope_cs(ang, c, sn);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float c, sn;
-      rope_cs(r, pos, d0 / 2 + i, c, sn);
       const float a = x[2 * i], b = x[2 * i + 1];
-      x[2 * i] = a * c - b * sn;
-      x[2 * i + 1] = a * sn + b * c;
+      x[2 * i] = a * c[i] - b * sn[i];
+      x[2 * i + 1] = a * sn[i] + b * c[i];
     }
   } else {
     const int half = r.dims / 2;
     const bool lo = d0 < half;
+    float ang[8], c[8], sn[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float c, sn;
-      rope_cs(r, pos, (lo ? d0 : d0 - half) + e, c, sn);
-      x[e] = lo ? x[e] * c - xp[e] * sn : x[e] * c + xp[e] * sn;
-    }
+    for (int e = 0; e < 8; ++e) ang[e] = rope_angle(r, pos, (lo ? d0 : d0 - half) + e);
+    rope_cs(ang, c, sn);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = lo ? x[e] * c[e] - xp[e] * sn[e] : x[e] * c[e] + xp[e] * sn[e];
   }
 }
 
@@ -124,6 +166,7 @@ struct RowMap {
   uint32_t total, L, H, per_row;
   Div31 div_c, div_l, div_h;
   int64_t l0;
+  int codes16;  // the code rows of both jobs are 16-byte aligned: 4 words a store
 };
 
 // Paged destination: row r of sequence b goes to row r % 64 of page table[b][r / 64] (the job's
@@ -247,8 +290,21 @@ __global__ __launch_bounds__(256) void quantize_append_kernel(QuantJob job0, Qua
   // the codes stay bit-identical and the division is the rare path.
   constexpr int W = kEPT * BITS / 32 > 0 ? kEPT * BITS / 32 : 1;  // code words per thread (2-bit, 8 elements: half a word)
   uint32_t packed[W];
+  float low = 0.0f;  // 4 bits: the code before, the low nibble of its byte
   auto put = [&](int i, float c) {
+    if constexpr (BITS == 8) {
+      // one instruction clamps to [0, 255] (NaN to 0, as below), converts and inserts the byte
+      packed[i / 4] = __builtin_amdgcn_cvt_pk_u8_f32(c, i % 4, i % 4 == 0 ? 0u : packed[i / 4]);
+      return;
+    }
     c = fminf(fmaxf(c, 0.0f), n_bins);
+    if constexpr (BITS == 4) {  // a byte is low + 16 c, exact
+      if (i % 2)
+        packed[i / 8] = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_fmaf(c, 16.0f, low), i / 2 % 4,
+                                                       i % 8 == 1 ? 0u : packed[i / 8]);
+      low = c;
+      return;
+    }
     const int bit = i * BITS;
     if (bit % 32 == 0) packed[bit / 32] = 0u;
     packed[bit / 32] |= (uint32_t)c << (bit % 32);
@@ -284,6 +340,10 @@ __global__ __launch_bounds__(256) void quantize_append_kernel(QuantJob job0, Qua
   if constexpr (kEPT * BITS < 32) {  // 2-bit, 8 elements: 16 bits; two neighbouring threads share a word
     const uint32_t other = (uint32_t)__builtin_amdgcn_ds_bpermute((__lane_id() ^ 1) << 2, (int)packed[0]);
     if ((chunk & 1) == 0) cdst[chunk / 2] = packed[0] | (other << 16);
+  } else if (W % 4 == 0 && rm.codes16) {  // 16-byte aligned rows
+#pragma unroll
+    for (int w = 0; w + 3 < W; w += 4)
+      *(u4*)(cdst + chunk * W + w) = u4{packed[w], packed[w + 1], packed[w + 2], packed[w + 3]};
   } else if constexpr (BITS == 8) {  // 8-byte aligned (checked on the host)
 #pragma unroll
     for (int w = 0; w < W; w += 2) *(u2*)(cdst + chunk * W + w) = u2{packed[w], packed[w + 1]};
@@ -307,8 +367,10 @@ template <typename T, int BITS, int G>
 static hipError_t launch_quant(const QuantJob& k, const QuantJob& v, int njobs, int B, int H, int L, int D,
                                int64_t row_offset, const RopeArgs* rope, const PageMap& pm, hipStream_t stream) {
   // rows per launch: the thread index of every launch stays below 2^31 (more rows take more launches)
-  // 32 elements per thread when that launch still has 8 or more workgroups per CU (2048 in all)
-  const bool wide = (int64_t)B * H * L * (D / 32) * njobs >= 2048 * 256;
+  // 32 elements per thread where that launch still has 2 workgroups per CU (512 in all), 4 with the rotation,
+  // whose longer threads need more of them in flight: without it 1024 rows of 8 heads of 256 dims (8-bit, 512
+  // workgroups) take 6.9 us at 8 elements and 5.3 at 32, with it 9.8 and 9.9, and 2048 rows 16.4 and 13.3
+  const bool wide = (int64_t)B * H * L * (D / 32) * njobs >= (rope ? 1024 : 512) * 256;
   const int ept = wide ? 32 : 8;
   const int64_t per_l = (int64_t)B * H * (D / ept);
   if (per_l >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
@@ -317,6 +379,10 @@ static hipError_t launch_quant(const QuantJob& k, const QuantJob& v, int njobs, 
   rm.H = (uint32_t)H;
   rm.div_h = make_div31((uint32_t)H);
   rm.per_row = (uint32_t)(D / ept);
+  rm.codes16 = 1;
+  for (const QuantJob* j : {&k, &v})
+    if (j == &k || njobs > 1)
+      rm.codes16 &= (uintptr_t)j->codes % 16 == 0 && (j->c_b | j->c_h | j->c_s) % 4 == 0;
   rm.div_c = make_div31(rm.per_row);
   for (int64_t l0 = 0; l0 < L; l0 += max_l) {
     const int64_t nl = L - l0 < max_l ? L - l0 : max_l;

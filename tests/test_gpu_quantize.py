@@ -163,3 +163,18 @@ def test_quantize_counterpart_of_mx_quantize():
     rc, rs, rb = OQ.quantize(to_np_bits(x), "float16", 64, 4)
     assert np.array_equal(c.cpu().view(torch.int32).numpy().view(np.uint32), rc)
     assert np.array_equal(to_np_bits(s), rs) and np.array_equal(to_np_bits(b), rb)
+
+
+@pytest.mark.parametrize("bits,pad", [(8, 2), (8, 4), (4, 1), (4, 2), (4, 4), (2, 1)])
+@pytest.mark.parametrize("L", [37, 1100])  # 8 and 32 elements a thread (1100 rows of 8 heads of 128: 550 workgroups)
+def test_code_rows_of_every_alignment(bits, pad, L):
+    # code rows a few words into wider ones: 16-byte stores only where every row allows them
+    print(f"quantize bits={bits} rows {pad} words into wider ones, L={L}", flush=True)
+    B, H, D, G = 2, 8, 128, 64
+    x = _stress((B, H, L, D), 77 + bits, torch.float16)
+    _, scales, biases = _alloc(B, H, L + 2, D, bits, G, torch.float16)
+    wide = torch.zeros((B, H, L + 2, D * bits // 32 + pad), dtype=torch.int32, device=DEV)
+    dst = (wide[..., pad:].view(torch.uint32), scales, biases)
+    kernels.quantize_append(x, dst, row_offset=1, group_size=G, bits=bits)
+    _check_rows(x, dst, 1, bits, G)
+    assert int(wide[..., :pad].abs().sum()) == 0 and int(wide[:, :, [0, L + 1]].abs().sum()) == 0

@@ -1,8 +1,8 @@
 """GPU RoPE: the in-place query rotation (kvq_rope) against the CPU restatement, and the fused
 rotate-and-quantize append (kvq_rope_quantize_append) against quantizing the rotated keys.
 
-Tolerance of the rotation: the GPU takes sin/cos of the fp32 angle with the device's fp32
-sincosf (within about 1 fp32 ulp), the restatement takes the correctly rounded values, so a
+Tolerance of the rotation: the GPU takes sin/cos of the fp32 angle in fp32 (within about 1 fp32
+ulp), the restatement takes the correctly rounded values, so a
 rotated element may round to a neighbouring value of its dtype. Each element must lie within one
 ulp of its dtype (plus 2^-22 of the row's largest input, for cancellation in a*cos - b*sin) and at
 most 0.2% of the elements may differ at all. The fused append must store exactly what quantizing
@@ -72,6 +72,20 @@ def test_rope_in_place_vs_oracle(dtype, case):
     x[0, 1, 3] *= 30.0
     y = x.to(DEV)
     assert kernels.rope(y, r, offset) is y
+    torch.cuda.synchronize()
+    _assert_rope_close(y, x, r, offset, "rope")
+
+
+@pytest.mark.parametrize("trad", [False, True])
+@pytest.mark.parametrize("offset", [131071, 2**26 - 30, 2**26 + 64, 2**31])
+def test_rope_far_positions(trad, offset):
+    # both reductions of the angle (the line is 2^26 rad, here crossed within a row's pairs, at 2^26 - 30
+    # within the rows): the angle is the same fp32 number on both sides, so the bound is the one above
+    print(f"rope far positions offset={offset} traditional={trad}", flush=True)
+    r = kernels.Rope(128, trad, 10000.0, 1.0)
+    x = seeded_normal((1, 3, 60, 128), 17, torch.float16)
+    y = x.to(DEV)
+    kernels.rope(y, r, offset)
     torch.cuda.synchronize()
     _assert_rope_close(y, x, r, offset, "rope")
 
