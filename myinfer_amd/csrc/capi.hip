@@ -342,9 +342,9 @@ size_t kvq_decode_workspace_size(int B, int Hq, int Hkv, int L, int D, int S, in
   // and every scale-group size (the group sets the query rows per workgroup)
   const int Dk = kvq::decode_kernel_dim(D);
   size_t n = 0;
-  for (int bits : {8, 4, 16})
+  for (int bits : {8, 16})  // (4 bits plan as 8 do; every unquantized plan is that of group 64)
     for (int G : {32, 64, 128}) {
-      if (G > Dk || 4 * G < Dk || (bits == 16 && Dk > 128)) continue;
+      if (G > Dk || 4 * G < Dk || (bits == 16 && (Dk > 128 || G != 64))) continue;
       const size_t x = kvq::decode_workspace_bytes(B, Hq, Hkv, L, D, S, window, bits, G);
       n = x > n ? x : n;
     }
@@ -565,10 +565,10 @@ int kvq_decode_attn_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qt
                            int Hq, int Hkv, int L, int D, int S, int bits, int group_size, int dtype, float scale,
                            const kvq_mask* mask, void* workspace, size_t workspace_bytes, void* stream) {
   if (check_head_dim(D, "decode")) return KVQ_ERR_UNSUPPORTED;
-  int rc = check_attn(q, k, v, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale, 0,
-                      kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0), workspace, workspace_bytes);
-  if (rc || (rc = check_mask(mask))) return rc;
   const size_t ws = kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0);
+  int rc = check_attn(q, k, v, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale, 0, ws, workspace,
+                      workspace_bytes);
+  if (rc || (rc = check_mask(mask))) return rc;
   if (masked_on_prefill(k, v, out, B, Hq, Hkv, L, D, S, group_size, dtype, mask, ws))
     return hip_status(kvq::launch_prefill_masked(q, k, v, nullptr, nullptr, out, B, Hq, Hkv, L, D, S, bits, group_size,
                                                  dtype, scale, mask, workspace, ws, (hipStream_t)stream),

@@ -3,7 +3,6 @@
 #include <stdlib.h>
 
 #include <algorithm>
-#include <numeric>
 
 #include "decode_kernel.h"
 
@@ -52,22 +51,22 @@ DecPlan decode_plan(int B, int Hq, int Hkv, int L, int D, int S, int window, int
   const int nrows = (Hq / Hkv) * L;
   pl.rowblocks = (nrows + pl.R - 1) / pl.R;
   pl.span = window > 0 ? std::min(S, window + L - 1 + kTile - 1) : S;  // the window, from a tile boundary
-  const int64_t tiles_seq = (pl.span + kTile - 1) / kTile;
+  const int tiles_seq = (pl.span + kTile - 1) / kTile;
   pl.nunits = B * Hkv * pl.rowblocks;
   // as many splits as the target holds whole: a unit count that does not divide 256 would otherwise leave a
   // few workgroups to run after the others. With the count rounded up instead, 32768 8-bit keys of 24, 40
   // and 72 units took 53.0, 88.7 and 151.9 us; so 41.6, 64.3 and 111.8. Where it costs the workgroups no
   // length (or little, and row blocks share keys) the count also makes the grid a multiple of the XCDs,
   // which keeps a unit's splits, and the row blocks of a key range, on one
-  auto tiles_of = [&](int64_t n) {
-    const int64_t t = (tiles_seq + n - 1) / n;
-    return std::max<int64_t>(pl.nw, (t + pl.nw - 1) / pl.nw * pl.nw);
+  auto tiles_of = [&](int n) {
+    const int t = (tiles_seq + n - 1) / n;
+    return std::max(pl.nw, (t + pl.nw - 1) / pl.nw * pl.nw);
   };
-  int64_t ns = std::max<int64_t>(1, std::min<int64_t>(tune.target_wgs / pl.nunits, kMaxSplit));
-  const int64_t whole = kXcds / std::gcd(pl.nunits, kXcds);
-  int64_t tpw = tiles_of(ns);
+  const int ns = std::max(1, std::min<int>(tune.target_wgs / pl.nunits, kMaxSplit));
+  const int whole = std::max(1, kXcds / (pl.nunits & -pl.nunits));  // (kXcds is a power of two)
+  int tpw = tiles_of(ns);
   if (ns > whole && 8 * tiles_of(ns - ns % whole) <= (pl.rowblocks > 1 ? 9 : 8) * tpw) tpw = tiles_of(ns - ns % whole);
-  pl.chunk = (int)(tpw * kTile);
+  pl.chunk = tpw * kTile;
   pl.nsplit = (pl.span + pl.chunk - 1) / pl.chunk;
   const bool fused = tune.fused < 0 ? pl.nsplit <= kFusedMaxSplit : tune.fused != 0;
   // (with 16 query rows of 128 dims a thread owns two float4s of a partial; the in-kernel merge

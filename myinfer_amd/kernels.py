@@ -307,7 +307,8 @@ NATIVE_HEAD_DIMS = (64, 128, 256)
 def kernel_dim(D: int) -> int:
     """The width the kernels compute head dimension D at: 64, 128 or 256. Other multiples of 8 (up to
     256 for quantized caches, 128 for unquantized ones) run the decode kernel at the next width, with
-    zero queries past their last dim, for every query length."""
+    zero queries past their last dim, for every query length (quantized 96 up to 64 rows: past them
+    the prefill kernel has a 96-wide form)."""
     return 64 if D <= 64 else 128 if D <= 128 else 256
 
 
@@ -599,8 +600,9 @@ def masked_attention(queries: torch.Tensor, keys, values, scale: float, mask: to
                      group_size: int = 64, bits: int = 8, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """softmax(scale * q K^T + mask) V under a general mask (boolean: visible keys; float: added to
     the scores), keys/values quantized triples or unquantized tensors as for ``attention``. Runs the
-    decode kernel (any L: rows beyond one pass take more passes over the keys), or, for an
-    unquantized head_dim-256 cache, the head_dim-256 kernel. A row that sees no key returns 0."""
+    decode kernel (rows beyond one pass take more passes over the keys), the prefill kernel where it
+    has the mask's form (boolean, and additive over unquantized caches) and the rows and keys are
+    many, or, for an unquantized head_dim-256 cache, the head_dim-256 kernel. A row that sees no key returns 0."""
     if queries.dim() != 4:
         raise ValueError(f"queries must be [B, Hq, L, D], got {tuple(queries.shape)}")
     B, Hq, L, D = queries.shape
@@ -645,8 +647,12 @@ def masked_attention(queries: torch.Tensor, keys, values, scale: float, mask: to
                                               B, Hq, Hkv, L, D, S, _lib.dtype_code(queries.dtype), *tail)
         _lib.check(rc, "kvq_decode_attn_dense_masked")
     else:
-        kq = _lib.qtensor(*keys, range_exp=range_word(keys[0]))
-        vq = _lib.qtensor(*values, range_exp=range_word(values[0]))
+        # a bf16 cache's range words, which only the prefill kernel reads; without them a call stays on the
+        # decode kernel, so finding them (3 us) waits for the sizes past which the library takes the other
+        passes = -(-(Hq // Hkv * L) // (4 if D == 96 else max(1, 1024 // D)))
+        words = queries.dtype == torch.bfloat16 and passes * B * Hkv * S >= 400_000
+        kq = _lib.qtensor(*keys, range_exp=range_word(keys[0]) if words else None)
+        vq = _lib.qtensor(*values, range_exp=range_word(values[0]) if words else None)
         rc = lib.kvq_decode_attn_masked(ctypes.byref(qr), ctypes.byref(kq), ctypes.byref(vq), ctypes.byref(orr), B, Hq,
                                         Hkv, L, D, S, int(bits), int(group_size), _lib.dtype_code(queries.dtype), *tail)
         _lib.check(rc, "kvq_decode_attn_masked")
