@@ -32,8 +32,9 @@ Masks (the reference accepts None, a string, or an array):
                         batch row (keys >= S_b masked), is recognised and runs as that structure;
                         any other boolean mask (per-head masks included) is read by the kernel
   additive float        all-zero runs unmasked; any other is added to the scores by the kernel
-General masks (kernels.masked_attention) run on the decode kernel for any L, broadcast as the
-reference broadcasts them on the same path; a row that sees no key returns 0.
+General masks (kernels.masked_attention) run on the decode kernel, or on the prefill kernel where
+there are many rows and keys, broadcast as the reference broadcasts them on the same path; a row
+that sees no key returns 0.
 Keyword extensions: ``window=`` (sliding window) and ``seq_lens=`` (int32 [B] valid key counts)
 give the same structure without building a mask.
 """
