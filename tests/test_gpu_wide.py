@@ -3,7 +3,7 @@
 Head_dim 256 is the Gemma family's width (Gemma-2 and the smaller Gemma-3 models). The kernel
 serves prefill over quantized caches (4/8-bit, groups 64 and 128) and every call, decode included,
 over unquantized caches (the plain cache before quantized_kv_start and the sliding-window layers).
-At head_dim 64 (Llama-3.2-1B, Qwen2.5-0.5B) it serves prefill over unquantized caches.
+Unquantized head_dim 64 (Llama-3.2-1B, Qwen2.5-0.5B) is checked here too; its prompts run on the prefill kernel.
 Covers GQA ratios, causal / full / sliding-window masks, variable-length batches, ragged query and
 key counts (partial tiles and row blocks, row blocks spanning two heads), capacity-padded views,
 split key ranges merged by combine_kernel, a Gemma-3-12B prefill chunk, and the public API's
