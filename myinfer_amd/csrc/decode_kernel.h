@@ -48,7 +48,6 @@
 namespace kvq {
 
 constexpr int kTile = 32;
-constexpr int kXcds = 8;
 
 // BITS == 16 is the unquantized cache: raw T rows, no scales or biases. It keeps the column
 // layout of the quantized cache (R query rows, each in NG columns), with every column computing the

@@ -14,19 +14,9 @@
 #include <math.h>
 
 #include "common.h"
+#include "limits.h"
 
 namespace kvq {
-
-constexpr int kMaxSplit = 128;
-
-// Launches whose last-arriving workgroup merges the splits count arrivals per unit in a counter
-// block at the start of the workspace. Every launch reserves the same block, so launches of
-// different shapes that share one workspace never place partials over another launch's counters;
-// a launch with more units than this does not split (prefill) or merges with combine_kernel
-// (decode). Counters start at zero (the workspace is zero-filled once) and the merging workgroup
-// resets its own.
-constexpr int kMaxCountedUnits = 65536;
-constexpr size_t kCounterBytes = (size_t)kMaxCountedUnits * sizeof(unsigned);
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll

@@ -6,74 +6,6 @@
 
 namespace kvq {
 
-struct PrePlan {
-  int rowblocks, nunits, nsplit, chunk, longest_first;
-};
-
-// Splits merged by the last of them to arrive; more take prefill_combine_kernel. Few splits are cheaper
-// in the kernel (the last 512-token chunk of 16384, 4 splits: 155.2 against 161.3 us for the layer
-// step), many in a launch of their own, whose loads run side by side: 64 rows of 4 KV heads over 8192
-// keys (32 splits) 45.5 -> 18.4 us, over 32768 (64 splits) 81.2 -> 28.0.
-constexpr int kPFusedMaxSplit = 4;
-
-static PrePlan prefill_plan(int B, int Hq, int Hkv, int L, int S, int window, int causal) {
-  PrePlan pl;
-  const int rep = Hq / Hkv, nrows = rep * L;
-  pl.rowblocks = (nrows + kPRows - 1) / kPRows;
-  pl.nunits = B * Hkv * pl.rowblocks;
-  // keys a row block sees: the whole context, or about a window; the first row block of a causal call
-  const int span = window > 0 ? std::min(S, window + kPRows) : S;
-  const int first = causal && window == 0 ? std::min(S, S - L + (kPRows + rep - 1) / rep) : span;
-  const int tiles = (span + kPT - 1) / kPT, tiles0 = (first + kPT - 1) / kPT;
-  const int nbk = B * Hkv;
-  const bool unequal = 2 * tiles0 <= tiles;
-  int ns = (kPTargetWgs + pl.nunits - 1) / pl.nunits;
-  if (unequal) {
-    // A causal prompt, whose first row blocks see few keys: the number of splits with the shortest
-    // estimate, in tiles (of about 2.2 us at 128 dims), of max(the longest workgroup, an even share of
-    // all work), a workgroup costing 4 tiles besides its own and 2 more where it takes part in a merge.
-    // 32 KV heads of 96 dims, 1999 tokens, 1 / 2 splits: 56 / 48 us; 4 KV heads of 8 query heads of
-    // 128 dims, 1000 tokens, 2 / 3 / 4 splits: 26.5 / 24.8 / 37.9 us.
-    const float avg = 0.5f * (tiles + tiles0);
-    float best = 0.0f;
-    for (int c = 1; c <= kPFusedMaxSplit; ++c) {
-      const int chunk = (tiles + c - 1) / c, cost = c > 1 ? 6 : 4;
-      const float total = pl.nunits * (avg + (avg / chunk + 0.5f) * cost);
-      const float est = std::max(total / kPTargetWgs, (float)(chunk + cost));
-      if (c == 1 || est < best) {
-        best = est;
-        ns = c;
-      }
-    }
-  }
-  ns = std::min(ns, std::max(1, tiles / 4));  // at least about 4 tiles per split
-  pl.nsplit = pl.nunits > kMaxCountedUnits ? 1 : std::max(1, std::min(ns, kMaxSplit));
-  pl.chunk = (tiles + pl.nsplit - 1) / pl.nsplit * kPT;
-  const bool dealt = nbk % kXcds == 0 ||
-                     (nbk < kXcds && kXcds % nbk == 0 && pl.rowblocks * pl.nsplit % (kXcds / nbk) == 0);
-  pl.longest_first = !unequal ? 0 : dealt ? 1 : 2;
-  return pl;
-}
-
-// Workspace: [arrival counters (the block shared with decode)][o partials][(m, l) partials]
-struct PreLayout {
-  size_t o, ml, total;
-};
-static PreLayout prefill_layout(const PrePlan& pl, int D) {
-  PreLayout l;
-  const size_t slots = (size_t)pl.nunits * pl.nsplit * kPRows;
-  l.o = kCounterBytes;
-  l.ml = l.o + slots * D * sizeof(uint16_t);  // fp16 rows
-  l.total = l.ml + (slots * 4 * sizeof(float) + 255) / 256 * 256;  // (m, l, 2^e, -) records
-  return l;
-}
-
-// The plan with as many splits as `bytes` of workspace hold (at 64 and 128 dims always all of them).
-static PrePlan fit_plan(PrePlan pl, int D, size_t bytes) {
-  while (pl.nsplit > 1 && prefill_layout(pl, D).total > bytes) --pl.nsplit;
-  return pl;  // (fewer splits take longer chunks: split_keys)
-}
-
 size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window, int) {
   size_t n = 256;
   for (int causal : {0, 1}) {
@@ -238,18 +170,15 @@ struct MaskedPlan {
 };
 static bool plan_masked(int B, int Hq, int Hkv, int L, int D, int S, const kvq_mask* mask, size_t bytes, MaskedPlan* m) {
   PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, 0, 0);
-  const int nbk = B * Hkv;
+  pl.unequal = true;  // most masks are causal and then some: the row blocks of the last positions first
+  set_splits(&pl, pl.nsplit);
   m->nwords = ((S + kPT - 1) / kPT + 63) / 64;
   const size_t need = (size_t)B * (mask->stride_kvh ? Hkv : 1) * pl.rowblocks * m->nwords * 16;
-  for (;; --pl.nsplit) {
+  for (;; set_splits(&pl, pl.nsplit - 1)) {
     m->words = pl.nsplit > 1 ? (prefill_layout(pl, D).total + 255) / 256 * 256 : kCounterBytes;
     if (m->words + need <= bytes) break;
     if (pl.nsplit == 1) return false;
   }
-  // most masks are causal and then some: the row blocks of the last positions first
-  const bool dealt = nbk % kXcds == 0 ||
-                     (nbk < kXcds && kXcds % nbk == 0 && pl.rowblocks * pl.nsplit % (kXcds / nbk) == 0);
-  pl.longest_first = dealt ? 1 : 2;
   m->pl = pl;
   return true;
 }

@@ -43,20 +43,17 @@
 #include "dma.h"
 #include "launch.h"
 #include "merge.h"
+#include "prefill_plan.h"
 
 namespace kvq {
 
-constexpr int kPT = 64;       // keys per tile
-constexpr int kPRows = 256;   // query rows per workgroup (8 waves x 32 MFMA columns)
 constexpr int kPW = 8;        // waves per workgroup
 // fp16 per K row in LDS: D + 8 (rows shift by 4 banks)
 template <int D>
 constexpr int kKS = D + 8;
 constexpr int kVS = 72;       // fp16 per V^T row in LDS: 64 + 8
 constexpr float kPSlack = 6.0f;
-constexpr int kPTargetWgs = 256;  // one workgroup per CU
 constexpr int kRawSlots = 3;
-constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 
 // The raw tile ring. A slot holds one 64-key tile as loaded: [K codes][V codes][sK, bK, sV, bV],
 // code rows with their 16-byte chunks permuted by row (chunk c of row r at position pos(r, c)), each
@@ -150,9 +147,9 @@ struct PreParams {
   float* part_o;
   float* part_ml;
   unsigned* counters;  // arrivals per unit, zero between launches
-  int xcd_remap;       // 1: the grid is a multiple of the XCD count (see the numbering in the kernel)
+  int xcd_remap;       // 1: the grid is a multiple of the XCD count (see prefill_wg)
   int longest_first;   // row blocks of unequal length, numbered from the longest down: 1 over all (sequence,
-                       // KV head) pairs of an XCD, 2 within each pair
+                       // KV head) pairs of an XCD, 2 within each pair (set_splits)
   int Hq, Hkv, L, S, rep, nrows, rowblocks, nsplit, nunits;
   int chunk;           // keys per split (a multiple of 64); see split_keys
   int fused;           // 1: the last split of a row block merges; 0: prefill_combine_kernel does
@@ -529,38 +526,8 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qc = lane & 31, hh = lane >> 5;
 
-  // Workgroup numbering: the row blocks of one (sequence, KV head, split) share every K/V tile, so
-  // they are consecutive, and consecutive workgroups are placed on one XCD (the hardware hands
-  // workgroups to the 8 XCDs in turn): each tile is fetched into one L2 rather than eight.
-  int rb, split, bk;  // bk = b * Hkv + kvh
-  if (p.longest_first == 1) {
-    // a causal prompt, whose last row blocks see many times the keys of its first: every XCD takes its
-    // share of the (sequence, KV head) pairs (or a pair's row blocks are dealt to several XCDs) and
-    // runs the row blocks of all of them from the longest down, so that short ones fill the end
-    const int x = blockIdx.x % kXcds, i = blockIdx.x / kXcds, nbk = (int)gridDim.x / (p.rowblocks * p.nsplit);
-    int rank;
-    if (nbk >= kXcds) {
-      const int mine = nbk / kXcds;
-      bk = x * mine + i % mine;
-      rank = i / mine;
-    } else {
-      const int per = kXcds / nbk;
-      bk = x / per;
-      rank = i * per + x % per;
-    }
-    rb = p.rowblocks - 1 - rank / p.nsplit;
-    split = rank % p.nsplit;
-  } else {
-    int wg = blockIdx.x;
-    if (p.xcd_remap) {
-      const int per_xcd = (int)(gridDim.x / kXcds);
-      wg = (wg % kXcds) * per_xcd + wg / kXcds;
-    }
-    rb = wg % p.rowblocks;
-    if (p.longest_first) rb = p.rowblocks - 1 - rb;
-    split = (wg / p.rowblocks) % p.nsplit;
-    bk = wg / (p.rowblocks * p.nsplit);
-  }
+  const PreWg wg = prefill_wg((int)blockIdx.x, (int)gridDim.x, p.rowblocks, p.nsplit, p.xcd_remap, p.longest_first);
+  const int rb = wg.rb, split = wg.split, bk = wg.bk;  // bk = b * Hkv + kvh
   const int b = bk / p.Hkv, kvh = bk % p.Hkv;
   const int unit = bk * p.rowblocks + rb;
   const int S_b = p.seq_lens ? min(max(load_uniform_i32(p.seq_lens, b), 0), p.S) : p.S;

@@ -11,6 +11,7 @@ import torch
 from myinfer_amd import kernels
 from tests.helpers import assert_close, exact_reference, seeded_normal
 from tests.test_gpu_decode import make_cache
+from tests.test_gpu_paged import build
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -76,3 +77,33 @@ def test_bf16_beyond_fp16():
     ref = exact_reference(q, kt, vt, 0.1, **kw)
     assert_close(kernels.attention(q, kt, vt, 0.1, **kw), ref, "one-shot")
     assert_close(kernels.prepare_attention(q, kt, vt, 0.1, **kw)(), ref, "prepared, no range word")
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,L,bits,dtype", [
+    (1, 32, 4, 975, 8, torch.float16),   # 31 row blocks of 4 pairs
+    (2, 8, 1, 1445, 4, torch.bfloat16),  # 46 of 2
+    (4, 5, 1, 1275, 8, torch.float16),   # 25 of 4
+    (1, 16, 4, 1600, 8, torch.bfloat16),
+    (1, 12, 4, 1904, 4, torch.float16),
+])
+def test_prompts_of_few_pairs(B, Hq, Hkv, L, bits, dtype, paged):
+    """Causal prompts of 2 or 4 (sequence, KV head) pairs, whose row blocks are dealt to the XCDs, at odd
+    numbers of row blocks and splits: every row is written and nothing before or after the output."""
+    print(f"prefill D=96 {B} {Hq} {Hkv} L={L} bits={bits} {dtype} paged={paged}", flush=True)
+    q = seeded_normal((B, Hq, L, D), 3401 + L, dtype, DEV)
+    scale = 1.0 / math.sqrt(D)
+    kw = dict(causal=True, group_size=G, bits=bits)
+    guard = 512 * D
+    buf = torch.full((2 * guard + q.numel(),), 7.0, dtype=dtype, device=DEV)
+    out = buf[guard:-guard].view(q.shape)
+    out.fill_(float("nan"))
+    if paged:
+        _, table, kp, vp, kt, vt = build(B, Hkv, [L] * B, D, bits, dtype, 3400 + L, group=G)
+        lens = torch.full((B,), L, dtype=torch.int32, device=DEV)
+        kernels.paged_attention(q, kp, vp, table, lens, scale, max_len=L, out=out, **kw)
+    else:
+        kt, vt = make_cache(B, Hkv, L, D, bits, dtype, 3400 + L, group=G)
+        kernels.attention(q, kt, vt, scale, out=out, **kw)
+    assert torch.all(buf[:guard] == 7.0) and torch.all(buf[-guard:] == 7.0)
+    assert_close(out, exact_reference(q, kt, vt, scale, **kw), f"L={L}")
