@@ -73,7 +73,8 @@ typedef struct kvq_rows {
  *     fp16 range still gives finite results (values below 2^(E - 24) then lose precision in the
  *     operands). E = 0 (or NULL) stages the values as they are: there a bf16 group beyond the fp16
  *     range makes the row blocks that read it return NaN, never a finite wrong value;
- *   - decode ignores it: it applies scales and biases in fp32.
+ *   - decode ignores it: it applies scales and biases in fp32. Its fp16 operand is a probability (up to
+ *     2^6) times a V scale; calls of one decode pass's rows need V scales up to 1023 for it.
  * This field has no counterpart in the reference, whose MLX kernels dequantize in bf16. */
 typedef struct kvq_qtensor {
   uint32_t* codes;

@@ -474,7 +474,8 @@ __device__ __forceinline__ h8 v_operand(const Bytes<VB> (&vc)[8], int jN) {
 
 // Rescaling slack, log2 units: a row's running maximum is raised only when a tile's maximum
 // exceeds it by more than this, so most tiles skip the accumulator rescale. Probabilities stay
-// below 2^kSlack; with fp16 scales (|s| <= 514) the fp16 PV operand p*s stays finite.
+// below 2^kSlack; with scales below 2^(16 - kSlack) (8-bit fp16 caches' are at most 514) the fp16 PV
+// operand p*s stays finite.
 constexpr float kSlack = 6.0f;
 
 // Split counts up to which the in-kernel merge loads every split's partial in one round.
@@ -810,20 +811,20 @@ __global__ __launch_bounds__(NW * 64, (dec_min_wgs<D, BITS, NW, NSLOT, G>())) vo
 #pragma unroll
     for (int s = 1; s < 8; ++s) tm = fmaxf(tm, sc[s]);
     tm = max_xor32(max_xor16(tm));
-    if (__builtin_amdgcn_ballot_w64(tm > m_run + kSlack) != 0) {
-      const float m_new = fmaxf(m_run, tm);
+    auto raise_max = [&](float m_new) {
       const float corr = (m_new == -INFINITY) ? 1.0f : exp2_fast(m_run - m_new);
       l_part *= corr;
       ob_part *= corr;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float ci = shfl(corr, (4 * lg + i) % R);
+        const float ci = shfl(corr, MULTI ? 4 * lg + i : (4 * lg + i) % R);
 #pragma unroll
         for (int jn = 0; jn < C::NBLK; ++jn) acc_o[jn][i] *= ci;
       }
       m_run = m_new;
-    }
-    const float msub = (m_run == -INFINITY) ? 0.0f : m_run;
+    };
+    if (__builtin_amdgcn_ballot_w64(tm > m_run + kSlack) != 0) raise_max(fmaxf(m_run, tm));
+    float msub = (m_run == -INFINITY) ? 0.0f : m_run;
     if constexpr (C::DENSE) {
       // P' (A operand) in the cache's type; the row sum adds the rounded probabilities, so the
       // output stays a convex combination of V rows whatever the rounding
@@ -843,36 +844,57 @@ __global__ __launch_bounds__(NW * 64, (dec_min_wgs<D, BITS, NW, NSLOT, G>())) vo
 #pragma unroll
       for (int jn = 0; jn < C::NBLK; ++jn) acc_o[jn] = mfma_16x16x32(aw, v_operand_dense(op.v, jn), acc_o[jn], T{});
     } else {
-      float pa[8];
-      float psum = 0.0f, pb = 0.0f;
+      u4 aw;
+      float psum, pb;
+      for (;;) {
+        float pa[8];
+        psum = pb = 0.0f;
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const float pr = exp2_fast(sc[s] - msub);
-        psum += pr;
-        pb += pr * sbv(3, s >> 2, s & 3);
-        pa[s] = pr * sbv(2, s >> 2, s & 3);
+        for (int s = 0; s < 8; ++s) {
+          const float pr = exp2_fast(sc[s] - msub);
+          psum += pr;
+          pb += pr * sbv(3, s >> 2, s & 3);
+          pa[s] = pr * sbv(2, s >> 2, s & 3);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          aw[a] = pack_f16x2(pa[2 * a], pa[2 * a + 1]);
+          if constexpr (MULTI) {
+            // what the fp16 operand dropped of p s multiplies codes that lie around the middle of their
+            // range: its product with the middle goes into the bias sum, so that only the codes' spread
+            // carries the rounding. Against 64 bits, fp16, 8 bits, 9006 keys: 2.8e-4 with it, 5.6e-4
+            // without, 4.6e-4 on the prefill kernel. (Halves are extracted with integer shifts: as
+            // elements of an h2 bit-cast from a u4 element the compiler, ROCm 7.2, reads all of them
+            // from one register in v_fma_mix_f32.)
+            const uint32_t w = aw[a];
+            const float lo = (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu));
+            const float hi = (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+            constexpr float kMid = (float)(1 << (BITS - 1));
+            pb = fmaf(kMid, pa[2 * a] - lo, pb);
+            pb = fmaf(kMid, pa[2 * a + 1] - hi, pb);
+          }
+        }
+        if constexpr (!MULTI) break;
+        // The operand p s reaches 2^kSlack times the scale, which a large scale takes past fp16 (bf16 caches of
+        // values beyond about 2.6e5 at 8 bits, fp16 caches of groups wider than 15000 at 4 bits); the sum above
+        // is then not finite. The prefill kernels that serve longer calls hold such caches, so here the column's
+        // maximum is raised until its largest product fits: what the operand then rounds away of the others is
+        // below 2^-38 of that one. (A product past fp32's range is left to become infinite. One pass's calls
+        // are left without this: it measured 2-4% of their time.)
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(fabsf(pb) < INFINITY)) == 0, 1)) break;
+        float pm = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) pm = fmaxf(pm, fabsf(pa[s]));
+        pm = max_xor32(max_xor16(pm));
+        const bool over = pm > 65504.0f && pm < INFINITY;
+        if (__builtin_amdgcn_ballot_w64(over) == 0) break;
+        int e = 15;
+        if (over) frexpf(pm, &e);  // pm < 2^e
+        raise_max(m_run + (float)(e - 15));
+        msub = (m_run == -INFINITY) ? 0.0f : m_run;
       }
       l_part += psum;
       ob_part += pb;
-      u4 aw;
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        aw[a] = pack_f16x2(pa[2 * a], pa[2 * a + 1]);
-        if constexpr (MULTI) {
-          // what the fp16 operand dropped of p s multiplies codes that lie around the middle of their
-          // range: its product with the middle goes into the bias sum, so that only the codes' spread
-          // carries the rounding. Against 64 bits, fp16, 8 bits, 9006 keys: 2.8e-4 with it, 5.6e-4
-          // without, 4.6e-4 on the prefill kernel. (Halves are extracted with integer shifts: as
-          // elements of an h2 bit-cast from a u4 element the compiler, ROCm 7.2, reads all of them
-          // from one register in v_fma_mix_f32.)
-          const uint32_t w = aw[a];
-          const float lo = (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu));
-          const float hi = (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
-          constexpr float kMid = (float)(1 << (BITS - 1));
-          ob_part = fmaf(kMid, pa[2 * a] - lo, ob_part);
-          ob_part = fmaf(kMid, pa[2 * a + 1] - hi, ob_part);
-        }
-      }
       const h8 aop = __builtin_bit_cast(h8, aw);
       // V codes of the lane's column slice at its 8 keys
       constexpr int VB = C::VLB < 2 ? 2 : C::VLB;
@@ -931,6 +953,14 @@ __global__ __launch_bounds__(NW * 64, (dec_min_wgs<D, BITS, NW, NSLOT, G>())) vo
   float obi[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) obi[i] = shfl(ob_part, 4 * lg + i);
+  float cf[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+  if constexpr (MULTI) {
+    // the columns of a row may hold their sums against maxima of their own: back to group 0's
+    const float m_row = shfl(m_run, n % R);
+    const float to_row = m_run == m_row ? 1.0f : exp2_fast(m_run - m_row);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cf[i] = shfl(to_row, 4 * lg + i);
+  }
   if (lg == 0 && n < R) {
     w_m[wave * R + n] = m_run;
     w_l[wave * R + n] = l_part;
@@ -947,7 +977,7 @@ __global__ __launch_bounds__(NW * 64, (dec_min_wgs<D, BITS, NW, NSLOT, G>())) vo
         if constexpr (BITS == 4) {
           if (jn & 1) x = (acc_o[jn][i] - acc_o[jn - 1][i]) * 1048576.0f;
         }
-        w_o[(wave * R + m % R) * D + (D / 16) * n + jn] = x + obi[i];
+        w_o[(wave * R + m % R) * D + (D / 16) * n + jn] = MULTI ? (x + obi[i]) * cf[i] : x + obi[i];
       }
     }
   }

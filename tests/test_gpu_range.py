@@ -7,7 +7,10 @@ kvq_qtensor.range_exp) that its appends raise, and the prefill kernels stage the
 2^-E and fold 2^E back into the scores (K) and the output (V). Through the cache objects and the
 drop-in entry points the results are finite and within the bars below; a raw prefill call whose
 descriptors carry no range word keeps the old policy: the row blocks that read such a group return
-NaN, never a finite wrong value. Decode applies scales and biases in fp32 and needs no scaling.
+NaN, never a finite wrong value. Decode applies scales and biases in fp32 and reads no word. Its PV
+operand, a probability times a value scale, is fp16: over more rows than one pass serves (the calls
+that prefill kernels serve at other sizes) the kernel raises the row's maximum where that would
+overflow; one pass's calls hold value scales up to 1023 (values to 2.6e5 at 8 bits).
 
 Bars: for values beyond the range, the bf16 bar (the fp16 V operands at 2^-E scale keep 11
 significant bits). For keys beyond the range the scores are large (about 1e4 to 1e5 in natural-log
@@ -196,6 +199,57 @@ def test_decode_exact_beyond_fp16():
     ref = exact_reference(q, kt, vt, scale, bits=bits)
     assert np.isfinite(out.cpu().float().numpy()).all()
     assert_close(out, ref, "decode beyond fp16")
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("D,rep,L", [(128, 2, 5), (128, 4, 10), (128, 4, 50), (64, 4, 20), (256, 2, 8)])
+def test_values_to_1e8_over_several_passes(bits, D, rep, L):
+    """Through the cache objects, contiguous and paged, with values of about 1e8 in one KV head and more rows
+    than a decode pass serves (p sV alone is beyond fp16)."""
+    print(f"range decode values bits={bits} D={D} rows={rep * L}", flush=True)
+    Hkv, S = 2, 900
+    k, v = big_rows(1, Hkv, S, D, 1, 1.0, 3e7, 360 + L)
+    cache = QuantizedKVCache(group_size=64, bits=bits)
+    kt, vt = cache.update_and_fetch(k, v)
+    q = seeded_normal((1, rep * Hkv, L, D), 361 + L, torch.bfloat16, DEV)
+    scale = 1.0 / math.sqrt(D)
+    causal = True
+    assert kernels.prepare_attention(q, kt, vt, scale, causal=causal, bits=bits).kernel == "decode"
+    out = A.blocked_quantized_sdpa(q, kt, vt, scale, "causal", 64, bits)
+    torch.cuda.synchronize()
+    for h in range(Hkv):  # a head at a time: the bars are of each head's own magnitude
+        part = [tuple(t[:, h:h + 1] for t in tr) for tr in (kt, vt)]
+        hs = slice(h * rep, (h + 1) * rep)
+        check_against_exact(out[:, hs], q[:, hs], *part, scale, bits, 0, f"head {h}", causal=causal)
+    pool = PagedRadixKVCache(1, Hkv, D, max_blocks=32, bits=bits, dtype=torch.bfloat16)
+    m = pool.match_and_allocate(list(range(S)), 16)
+    t = pool.tables([m.block_table])
+    pool.append(0, k, v, t)
+    lens = torch.tensor([S], dtype=torch.int32, device=DEV)
+    paged = kernels.paged_attention(q, pool.k_cache(0), pool.v_cache(0), t, lens, scale, causal=causal, bits=bits,
+                                    max_len=S)
+    assert torch.equal(paged, out)
+
+
+def test_wide_fp16_groups_behind_a_lagging_maximum():
+    """4-bit fp16 groups that span most of the type (scales of about 8000) and keys whose score is 5 (in log2
+    units) above the running maximum, which a wave does not raise for that: p sV reaches 2^18.
+    Bar: p sV rounded to fp16 against codes of mean square 8.6^2 whose spread is 4.4, 2^-11 / sqrt(3) x 2 =
+    5.6e-4 relative, and the output's rounding, 2.8e-4."""
+    print("range lagging maximum", flush=True)
+    B, Hkv, rep, L, S, D, bits = 2, 8, 2, 5, 6000, 128, 4
+    k = torch.zeros((B, Hkv, S, D))
+    k[:, :, 700::1000] = 1.083
+    v = 6e4 * (2 * torch.rand((B, Hkv, S, D), generator=torch.Generator().manual_seed(370)) - 1)
+    kt, vt = (kernels.quantize(x.half().to(DEV), 64, bits) for x in (k, v))
+    assert float(vt[1].abs().max()) > 7000
+    q = torch.full((B, rep * Hkv, L, D), 0.25, dtype=torch.float16, device=DEV)
+    out = kernels.attention(q, kt, vt, 0.1, bits=bits, kernel="decode")
+    ref = exact_reference(q, kt, vt, 0.1, bits=bits)
+    o = out.cpu().float().numpy().astype(np.float64)
+    assert np.isfinite(o).all()
+    st = OA.error_stats(o, ref)
+    assert st["rel_l2"] <= 1e-3, st
 
 
 def test_in_range_caches_are_unchanged():
