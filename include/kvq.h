@@ -244,8 +244,8 @@ int kvq_decode_attn_dense_masked(const kvq_rows* q, const kvq_rows* k, const kvq
  * ranges are merged by a second, small launch on the same stream. So are the other widths' where
  * more than 4 splits of a row block are merged. Head dim 96 runs the prefill kernel past 64 rows of a
  * KV head (Hq / Hkv * L), with D = 64's and 128's requirement on the output; where the output's
- * alignment or the workspace does not allow it, and at the other head dims, the decode kernel runs
- * (any L). All of these take kvq_decode_attn's workspace size.
+ * alignment does not allow it, and at the other head dims, the decode kernel runs (any L). The workspace
+ * is kvq_prefill_workspace_size's at every head dim.
  */
 int kvq_prefill_attn(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v,
                      const int32_t* seq_lens, const kvq_rows* out,

@@ -393,11 +393,12 @@ int kvq_decode_attn_static(const kvq_rows* q, const kvq_qtensor* k, const kvq_qt
 
 size_t kvq_prefill_workspace_size(int B, int Hq, int Hkv, int L, int D, int S, int window) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || S <= 0 || window < 0 || Hq % Hkv) return 0;
-  // the decode kernel serves; where the prefill kernel does (prefill_serves_96) its splits are fitted to
-  // the same size
-  if (!native_dim(D)) return kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, window);
+  if (!native_dim(D)) {  // the decode kernel serves, or at 96 dims the prefill kernel (prefill_serves_96)
+    const size_t n = kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, window);
+    return D == 96 && n ? std::max(n, kvq::prefill_workspace_bytes(B, Hq, Hkv, L, D, S, window)) : n;
+  }
   if (D == 256) return kvq::wide_workspace_bytes(B, Hq, Hkv, L, D, S, window);
-  return kvq::prefill_workspace_bytes(B, Hq, Hkv, L, D, S, window, 8);
+  return kvq::prefill_workspace_bytes(B, Hq, Hkv, L, D, S, window);
 }
 
 // The prefill kernel loads two scale groups of a row at once when a row has several: scale and
@@ -445,8 +446,7 @@ int kvq_prefill_attn(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor*
   if ((rc = check_rows(out, "out", D, true))) return rc;  // rows are stored 16 bytes at a time
   if (!at96 && (rc = check_prefill_sb(k, v, D, group_size))) return rc;
   return hip_status(kvq::launch_prefill(q, k, v, seq_lens, out, B, Hq, Hkv, L, D, S, bits, group_size, dtype, scale,
-                                        causal, window, workspace,
-                                        kvq_prefill_workspace_size(B, Hq, Hkv, L, D, S, window), (hipStream_t)stream),
+                                        causal, window, workspace, (hipStream_t)stream),
                     "prefill_attn launch");
 }
 
@@ -509,8 +509,7 @@ int kvq_paged_prefill_attn(const kvq_rows* q, const kvq_qtensor* k_pool, const k
   if (!at96 && (rc = check_prefill_sb(k_pool, v_pool, D, group_size))) return rc;
   return hip_status(kvq::launch_prefill_paged(q, k_pool, v_pool, num_pages, block_table, table_stride, seq_lens, out, B,
                                               Hq, Hkv, L, D, S, bits, group_size, dtype, scale, causal, window,
-                                              workspace, kvq_prefill_workspace_size(B, Hq, Hkv, L, D, S, window),
-                                              (hipStream_t)stream),
+                                              workspace, (hipStream_t)stream),
                     "paged_prefill_attn launch");
 }
 

@@ -40,19 +40,16 @@ hipError_t launch_decode_dense(const kvq_rows* q, const kvq_rows* k, const kvq_r
                                int causal, int window, void* workspace, hipStream_t stream,
                                const kvq_mask* mask = nullptr);
 
-size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window, int bits);
-// workspace_bytes: what the call's shapes entitle it to (kvq_prefill_workspace_size), which bounds the
-// key splits; not the size of the caller's buffer, so that a call's splits follow from its shapes
+size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window);
 hipError_t launch_prefill(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const int32_t* seq_lens,
                           const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype,
-                          float scale, int causal, int window, void* workspace, size_t workspace_bytes,
-                          hipStream_t stream);
+                          float scale, int causal, int window, void* workspace, hipStream_t stream);
 hipError_t launch_prefill_paged(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, int num_pages,
                                 const int32_t* table, int64_t table_stride, const int32_t* seq_lens, const kvq_rows* out,
                                 int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype, float scale,
-                                int causal, int window, void* workspace, size_t workspace_bytes, hipStream_t stream);
+                                int causal, int window, void* workspace, hipStream_t stream);
 // Under a general mask: bits 16 over kd / vd (head_dim 64 or 128), else over k / v (64, 96 or 128);
-// workspace_bytes as for launch_prefill.
+// workspace_bytes: what the call's shapes entitle it to, not the size of the caller's buffer.
 // prefill_masked_rows: whether the prefill kernel is the faster one for such a call; prefill_masked_bytes:
 // the workspace it would have then (0 else).
 bool prefill_masked_rows(int B, int Hq, int Hkv, int L, int D, int S);

@@ -6,11 +6,12 @@
 
 namespace kvq {
 
-size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window, int) {
+size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int window) {
   size_t n = 256;
   for (int causal : {0, 1}) {
     const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window, causal);
-    if (pl.nsplit > 1) n = std::max(n, prefill_layout(pl, D).total);
+    // (the size serves quantized and unquantized calls: at 64 dims the latter's partials are fp32)
+    if (pl.nsplit > 1) n = std::max(n, prefill_layout(pl, D, D != 128).total);
   }
   return n;
 }
@@ -21,7 +22,9 @@ static hipError_t launch_prefill_t(const PreParams& p, hipStream_t stream) {
                      p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.nsplit == 1 || p.fused) return e;
-  hipLaunchKernelGGL((prefill_combine_kernel<T, D>), dim3(p.nunits * kPW * (D / 16)), dim3(kPW * 64), 0, stream, p);
+  constexpr bool f32 = kF32Partials<BITS, D, 0>;
+  hipLaunchKernelGGL((prefill_combine_kernel<T, D, f32>), dim3(p.nunits * kPW * (D / (f32 ? 8 : 16))), dim3(kPW * 64), 0,
+                     stream, p);
   return hipGetLastError();
 }
 
@@ -55,7 +58,8 @@ static hipError_t launch_prefill_quant(const PreParams& p, int dtype, int D, int
 
 // Everything but the K/V operands.
 static PreParams prefill_params(const kvq_rows* q, const int32_t* seq_lens, const kvq_rows* out, int Hq, int Hkv, int L, int D,
-                                int S, float scale, int causal, int window, void* workspace, const PrePlan& pl) {
+                                int S, float scale, int causal, int window, void* workspace, const PrePlan& pl,
+                                bool f32_partials) {
   PreParams p{};
   p.q = (const uint16_t*)q->data;
   p.q_sb = q->stride_b;
@@ -66,7 +70,7 @@ static PreParams prefill_params(const kvq_rows* q, const int32_t* seq_lens, cons
   p.o_sb = out->stride_b;
   p.o_sh = out->stride_h;
   p.o_sl = out->stride_l;
-  const PreLayout lay = prefill_layout(pl, D);
+  const PreLayout lay = prefill_layout(pl, D, f32_partials);
   p.counters = (unsigned*)workspace;
   p.part_o = (float*)((char*)workspace + lay.o);
   p.part_ml = (float*)((char*)workspace + lay.ml);
@@ -125,10 +129,10 @@ static void dense_operands(PreParams& p, const kvq_rows* k, const kvq_rows* v) {
 
 hipError_t launch_prefill(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const int32_t* seq_lens,
                           const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype,
-                          float scale, int causal, int window, void* workspace, size_t workspace_bytes,
-                          hipStream_t stream) {
-  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window, causal), D, workspace_bytes);
-  PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
+                          float scale, int causal, int window, void* workspace, hipStream_t stream) {
+  const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window, causal);
+  PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl,
+                               D == 96);
   quant_operands(p, k, v);
   return launch_prefill_quant<false>(p, dtype, D, bits, G, stream);
 }
@@ -136,9 +140,10 @@ hipError_t launch_prefill(const kvq_rows* q, const kvq_qtensor* k, const kvq_qte
 hipError_t launch_prefill_paged(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, int num_pages,
                                 const int32_t* table, int64_t table_stride, const int32_t* seq_lens, const kvq_rows* out,
                                 int B, int Hq, int Hkv, int L, int D, int S, int bits, int G, int dtype, float scale,
-                                int causal, int window, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-  const PrePlan pl = fit_plan(prefill_plan(B, Hq, Hkv, L, S, window, causal), D, workspace_bytes);
-  PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
+                                int causal, int window, void* workspace, hipStream_t stream) {
+  const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window, causal);
+  PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl,
+                               D == 96);
   quant_operands(p, k, v);  // (batch strides are page strides)
   p.table = table;
   p.table_stride = table_stride;
@@ -150,7 +155,7 @@ hipError_t launch_prefill_dense(const kvq_rows* q, const kvq_rows* k, const kvq_
                                 const kvq_rows* out, int B, int Hq, int Hkv, int L, int D, int S, int dtype,
                                 float scale, int causal, int window, void* workspace, hipStream_t stream) {
   const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window, causal);
-  PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl);
+  PreParams p = prefill_params(q, seq_lens, out, Hq, Hkv, L, D, S, scale, causal, window, workspace, pl, D == 64);
   dense_operands(p, k, v);
   p.out8 = ((uintptr_t)out->data % 16 || (out->stride_b | out->stride_h | out->stride_l) % 8) ? 1 : 0;
   const bool bf = dtype == KVQ_DTYPE_BF16;
@@ -175,7 +180,7 @@ static bool plan_masked(int B, int Hq, int Hkv, int L, int D, int S, const kvq_m
   m->nwords = ((S + kPT - 1) / kPT + 63) / 64;
   const size_t need = (size_t)B * (mask->stride_kvh ? Hkv : 1) * pl.rowblocks * m->nwords * 16;
   for (;; set_splits(&pl, pl.nsplit - 1)) {
-    m->words = pl.nsplit > 1 ? (prefill_layout(pl, D).total + 255) / 256 * 256 : kCounterBytes;
+    m->words = pl.nsplit > 1 ? (prefill_layout(pl, D, true).total + 255) / 256 * 256 : kCounterBytes;
     if (m->words + need <= bytes) break;
     if (pl.nsplit == 1) return false;
   }
@@ -199,7 +204,7 @@ size_t prefill_masked_bytes(int B, int Hq, int Hkv, int L, int D, int S) {
   if (!prefill_masked_rows(B, Hq, Hkv, L, D, S)) return 0;
   const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, 0, 0);
   const size_t words = (size_t)B * Hkv * pl.rowblocks * (((S + kPT - 1) / kPT + 63) / 64) * 16;
-  return (pl.nsplit > 1 ? (prefill_layout(pl, D).total + 255) / 256 * 256 : kCounterBytes) + words;
+  return (pl.nsplit > 1 ? (prefill_layout(pl, D, true).total + 255) / 256 * 256 : kCounterBytes) + words;
 }
 
 bool prefill_masked_fits(int B, int Hq, int Hkv, int L, int D, int S, const kvq_mask* mask, size_t bytes) {
@@ -213,7 +218,7 @@ hipError_t launch_prefill_masked(const kvq_rows* q, const kvq_qtensor* k, const 
                                  size_t workspace_bytes, hipStream_t stream) {
   MaskedPlan m;
   if (!plan_masked(B, Hq, Hkv, L, D, S, mask, workspace_bytes, &m)) return hipErrorInvalidValue;
-  PreParams p = prefill_params(q, nullptr, out, Hq, Hkv, L, D, S, scale, 0, 0, workspace, m.pl);
+  PreParams p = prefill_params(q, nullptr, out, Hq, Hkv, L, D, S, scale, 0, 0, workspace, m.pl, true);
   if (bits == 16) {
     dense_operands(p, kd, vd);
   } else {

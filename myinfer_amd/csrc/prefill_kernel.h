@@ -501,6 +501,12 @@ __device__ __forceinline__ void stage_v_raw(const uint8_t* raw, _Float16* vlds, 
   *(u4*)&vlds[(2 * d2 + 1) * kVS + 8 * c8] = hi;
 }
 
+// Whether a split's partial rows are kept in fp32: for the calls that kernels with fp32 partials served before
+// this one (head_dim 96 and general masks the decode kernel, unquantized head_dim 64 the head_dim-256
+// kernel's form of that width). The others pack them to fp16, which their workspaces are sized for.
+template <int BITS, int D, int MASKED>
+constexpr bool kF32Partials = MASKED != 0 || D == 96 || (BITS == 16 && D == 64);
+
 // MASKED: 0, or under a general mask: 1 boolean, 2 additive. The tile loop then walks the list of tiles
 // with a visible key, and reads the mask beside those that are not visible as a whole.
 template <typename T, int BITS, bool PAGED = false, int G = 64, int D = 128, int MASKED = 0>
@@ -1142,16 +1148,25 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
     //    u (0 .. QW - 1) of 16 bytes at byte ((s * kPW + wave) * QW + u) * 1024 + 16 lane of the unit's o
     //    block; word u packs value groups 2u and 2u + 1 (group 4 db + c = oacc[db][4c .. 4c+3]).
     //    Record of row r at byte 16 (s * kPRows + r) of the unit's record block.
-    const __amdgpu_buffer_rsrc_t ro = make_rsrc((const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * (kPRows * 2 * D),
-                                                (uint32_t)p.nsplit * (kPRows * 2 * D));
+    //  * With fp32 partials (kF32Partials) a row is o itself, word u (0 .. 2 QW - 1) value group u, and its
+    //    record (m, l, 2^E_V): the merge scales row s by w_s 2^E_V.
+    constexpr bool F32P = kF32Partials<BITS, D, MASKED>;
+    constexpr int NW = F32P ? 2 * QW : QW;       // 16-byte words of a lane's row
+    constexpr uint32_t split_o = kPW * NW * 1024;
+    const __amdgpu_buffer_rsrc_t ro =
+        make_rsrc((const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * split_o, (uint32_t)p.nsplit * split_o);
     const __amdgpu_buffer_rsrc_t rm = make_rsrc(p.part_ml + (int64_t)unit * p.nsplit * (kPRows * 4),
                                                 (uint32_t)p.nsplit * (kPRows * 16));
-    const uint32_t lo = (uint32_t)wave * (QW * 1024) + 16 * lane;
-    const uint32_t split_o = kPW * QW * 1024;
+    const uint32_t lo = (uint32_t)wave * (NW * 1024) + 16 * lane;
     const uint32_t row_ml = 16 * (wave * 32 + qc);
-    u4 own[QW];
-    float own_sc;
-    {
+    f4 own[NW];
+    float own_sc = vback;  // the V operands were staged times 2^-E_V
+    if constexpr (F32P) {
+#pragma unroll
+      for (int g = 0; g < NW; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) own[g][i] = oacc[g >> 2][4 * (g & 3) + i];
+    } else {
       const float inv_l = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
       float mx = 0.0f;
 #pragma unroll
@@ -1164,19 +1179,22 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
       int ex = 0;
       if (mx > 0.0f) frexpf(mx, &ex);
       const int e = mx > 0.0f ? min(max(ex - 14, -100), 100) : 0;
-      own_sc = ldexpf(1.0f, e) * vback;  // the V operands were staged times 2^-E_V
+      own_sc *= ldexpf(1.0f, e);
       const float f = ldexpf(inv_l, -e);
 #pragma unroll
-      for (int u = 0; u < QW; ++u)
+      for (int u = 0; u < NW; ++u) {
+        u4 x;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int g = 2 * u + h, db = g >> 2, c = g & 3;
-          own[u][2 * h] = pack_f16x2(oacc[db][4 * c] * f, oacc[db][4 * c + 1] * f);
-          own[u][2 * h + 1] = pack_f16x2(oacc[db][4 * c + 2] * f, oacc[db][4 * c + 3] * f);
+          x[2 * h] = pack_f16x2(oacc[db][4 * c] * f, oacc[db][4 * c + 1] * f);
+          x[2 * h + 1] = pack_f16x2(oacc[db][4 * c + 2] * f, oacc[db][4 * c + 3] * f);
         }
+        own[u] = __builtin_bit_cast(f4, x);
+      }
     }
 #pragma unroll
-    for (int u = 0; u < QW; ++u) store_agent_b128(ro, lo + u * 1024 + split * split_o, __builtin_bit_cast(f4, own[u]));
+    for (int u = 0; u < NW; ++u) store_agent_b128(ro, lo + u * 1024 + split * split_o, own[u]);
     if (hh == 0) store_agent_b128(rm, row_ml + split * (kPRows * 16), f4{m_run, l_tot, own_sc, 0.0f});
     if (!p.fused) return;
     // The stores are acknowledged (written through to the device's coherence point) before the
@@ -1202,34 +1220,40 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
     float l_acc = 0.0f;
     for (int s2 = 0; s2 < nsplit; ++s2) {
       f4 rec;
-      u4 po[QW];
+      f4 po[NW];
       if (s2 == split) {
         rec = f4{m_run, l_tot, own_sc, 0.0f};
 #pragma unroll
-        for (int u = 0; u < QW; ++u) po[u] = own[u];
+        for (int u = 0; u < NW; ++u) po[u] = own[u];
       } else {
         rec = load_agent_b128(rm, row_ml, s2 * (kPRows * 16));
 #pragma unroll
-        for (int u = 0; u < QW; ++u) po[u] = __builtin_bit_cast(u4, load_agent_b128(ro, lo + u * 1024, s2 * split_o));
+        for (int u = 0; u < NW; ++u) po[u] = load_agent_b128(ro, lo + u * 1024, s2 * split_o);
       }
       const float w = (M == -INFINITY || rec[1] <= 0.0f) ? 0.0f : exp2_fast(rec[0] - M);
       l_acc = fmaf(w, rec[1], l_acc);
-      const float F = (w * rec[1]) * rec[2];
+      const float F = F32P ? w * rec[2] : (w * rec[1]) * rec[2];
 #pragma unroll
-      for (int u = 0; u < QW; ++u)
+      for (int u = 0; u < NW; ++u) {
+        if constexpr (F32P) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int g = 2 * u + h, db = g >> 2, c = g & 3;
-          // halves are extracted with integer shifts: converting the elements of an h2 bit-cast
-          // from a u4 element let the compiler (ROCm 7.2) fold all four words of a u4 into the
-          // first one's register in v_fma_mix_f32
+          for (int k = 0; k < 4; ++k) macc[u >> 2][4 * (u & 3) + k] = fmaf(F, po[u][k], macc[u >> 2][4 * (u & 3) + k]);
+        } else {
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const uint32_t w = po[u][2 * h + (k >> 1)];
-            const float x = (float)__builtin_bit_cast(_Float16, (uint16_t)((k & 1) ? w >> 16 : w & 0xffffu));
-            macc[db][4 * c + k] = fmaf(F, x, macc[db][4 * c + k]);
+          for (int h = 0; h < 2; ++h) {
+            const int g = 2 * u + h, db = g >> 2, c = g & 3;
+            // halves are extracted with integer shifts: converting the elements of an h2 bit-cast
+            // from a u4 element let the compiler (ROCm 7.2) fold all four words of a u4 into the
+            // first one's register in v_fma_mix_f32
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t w = __builtin_bit_cast(u4, po[u])[2 * h + (k >> 1)];
+              const float x = (float)__builtin_bit_cast(_Float16, (uint16_t)((k & 1) ? w >> 16 : w & 0xffffu));
+              macc[db][4 * c + k] = fmaf(F, x, macc[db][4 * c + k]);
+            }
           }
         }
+      }
     }
     l_tot = l_acc;
 #pragma unroll
@@ -1286,12 +1310,14 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
 // last split loads the others one after another (about 0.9 us each at 128 dims). A workgroup takes one
 // 16-byte word u of the packed rows of one wave (32 rows) of a row block; its 8 waves take the splits
 // in turn, four in flight each, and wave 0 sums the eight partial merges. Row blocks that were not
-// split have been written already.
-template <typename T, int D, bool MASKED = false>
+// split have been written already. F32P: the partials are fp32 (kF32Partials), a word 4 values of a row rather than 8.
+template <typename T, int D, bool F32P, bool MASKED = false>
 __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) {
-  constexpr int QW = D / 16;
+  constexpr int QW = F32P ? D / 8 : D / 16;  // words per row
+  constexpr int NV = F32P ? 4 : 8;           // values per word
+  constexpr int split_o = kPW * QW * 1024;
   __shared__ float s_m[kPW][64], s_l[kPW][64];
-  __shared__ __align__(16) float s_o[kPW][64][8];
+  __shared__ __align__(16) float s_o[kPW][64][NV];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int u = blockIdx.x % QW, w = (blockIdx.x / QW) % kPW, unit = blockIdx.x / (QW * kPW);
@@ -1308,10 +1334,10 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
     ks.nsplit = split_keys(p, S_b, fr0, frl).nsplit;
   }
   if (ks.nsplit == 1 || fr0 + 32 * w >= p.nrows) return;
-  const uint8_t* po = (const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * (kPRows * 2 * D) + (w * QW + u) * 1024 + 16 * lane;
+  const uint8_t* po = (const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * split_o + (w * QW + u) * 1024 + 16 * lane;
   const f4* rec = (const f4*)(p.part_ml + (int64_t)unit * p.nsplit * (kPRows * 4)) + 32 * w + (lane & 31);
   constexpr int CH = 4;
-  float M = -INFINITY, l = 0.0f, acc[8] = {};
+  float M = -INFINITY, l = 0.0f, acc[NV] = {};
   for (int s0 = wave; s0 < ks.nsplit; s0 += kPW * CH) {
     f4 r[CH];
     u4 v[CH];
@@ -1319,7 +1345,7 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
     for (int i = 0; i < CH; ++i) {
       const int s = min(s0 + kPW * i, ks.nsplit - 1);  // past the last split it is re-read, and not counted
       r[i] = rec[s * kPRows];
-      v[i] = *(const u4*)(po + (int64_t)s * (kPRows * 2 * D));
+      v[i] = *(const u4*)(po + (int64_t)s * split_o);
     }
     float Mn = M;
 #pragma unroll
@@ -1328,26 +1354,27 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
     const float corr = M == Mn ? 1.0f : exp2_fast(M - Mn);
     l *= corr;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] *= corr;
+    for (int e = 0; e < NV; ++e) acc[e] *= corr;
     M = Mn;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       if (s0 + kPW * i >= ks.nsplit) continue;
       // a row that saw no key in the split counts 0, but for NaN (a poisoned row block)
-      const float wl = r[i][1] > 0.0f ? exp2_fast(r[i][0] - M) * r[i][1] : 0.0f;
-      l += wl;
-      const float F = wl * r[i][2];
+      const float ws = r[i][1] > 0.0f ? exp2_fast(r[i][0] - M) : 0.0f;
+      l += ws * r[i][1];
+      const float F = (F32P ? ws : ws * r[i][1]) * r[i][2];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t x = v[i][e >> 1];
-        acc[e] = fmaf(F, (float)__builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? x >> 16 : x & 0xffffu)), acc[e]);
+      for (int e = 0; e < NV; ++e) {
+        const uint32_t x = v[i][F32P ? e : e >> 1];
+        acc[e] = fmaf(F, F32P ? __uint_as_float(x)
+                              : (float)__builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? x >> 16 : x & 0xffffu)), acc[e]);
       }
     }
   }
   s_m[wave][lane] = M;
   s_l[wave][lane] = l;
 #pragma unroll
-  for (int e = 0; e < 8; e += 4) *(f4*)&s_o[wave][lane][e] = f4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
+  for (int e = 0; e < NV; e += 4) *(f4*)&s_o[wave][lane][e] = f4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
   __syncthreads();
   const int row = fr0 + 32 * w + (lane & 31);
   if (wave != 0 || row >= p.nrows) return;
@@ -1355,21 +1382,21 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
 #pragma unroll
   for (int k = 0; k < kPW; ++k) M = fmaxf(M, s_m[k][lane]);
   l = 0.0f;
-  f4 o[2] = {};
+  f4 o[NV / 4] = {};
 #pragma unroll
   for (int k = 0; k < kPW; ++k) {
     const float f = s_m[k][lane] == -INFINITY ? (M == -INFINITY ? 1.0f : 0.0f) : exp2_fast(s_m[k][lane] - M);
     l += f * s_l[k][lane];
-    o[0] += f * *(const f4*)&s_o[k][lane][0];
-    o[1] += f * *(const f4*)&s_o[k][lane][4];
+#pragma unroll
+    for (int h = 0; h < NV / 4; ++h) o[h] += f * *(const f4*)&s_o[k][lane][4 * h];
   }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  // word u packs value groups 2u and 2u + 1; group 4 db + c holds dims 32 db + 8 c + 4 hh .. + 3
+  // word u holds value groups NV / 4 u ..; group 4 db + c holds dims 32 db + 8 c + 4 hh .. + 3
   uint16_t* dst = p.out + (int64_t)b * p.o_sb + (int64_t)(kvh * p.rep + row % p.rep) * p.o_sh +
                   (int64_t)(row / p.rep) * p.o_sl + 4 * (lane >> 5);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int g = 2 * u + h;
+  for (int h = 0; h < NV / 4; ++h) {
+    const int g = NV / 4 * u + h;
     u2 x;
     x[0] = (uint32_t)from_float(o[h][0] * inv, T{}) | ((uint32_t)from_float(o[h][1] * inv, T{}) << 16);
     x[1] = (uint32_t)from_float(o[h][2] * inv, T{}) | ((uint32_t)from_float(o[h][3] * inv, T{}) << 16);

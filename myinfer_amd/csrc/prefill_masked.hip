@@ -114,7 +114,7 @@ static hipError_t launch_t(const PreParams& p, hipStream_t stream) {
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.nsplit == 1 || p.fused) return e;
-  hipLaunchKernelGGL((prefill_combine_kernel<T, D, true>), dim3(p.nunits * kPW * (D / 16)), block, 0, stream, p);
+  hipLaunchKernelGGL((prefill_combine_kernel<T, D, true, true>), dim3(p.nunits * kPW * (D / 8)), block, 0, stream, p);
   return hipGetLastError();
 }
 

@@ -27,8 +27,8 @@ struct PrePlan {
 // keys (32 splits) 45.5 -> 18.4 us, over 32768 (64 splits) 81.2 -> 28.0.
 constexpr int kPFusedMaxSplit = 4;
 
-// Cut `pl` into `nsplit` splits. What follows from the count is set here and nowhere else, so that a plan
-// whose count is lowered (to fit a workspace) is numbered for the count it runs with.
+// Cut `pl` into `nsplit` splits. What follows from the count is set here and nowhere else, so that every plan is
+// numbered for the count it runs with.
 inline void set_splits(PrePlan* pl, int nsplit) {
   pl->nsplit = nsplit;
   pl->chunk = (pl->tiles + nsplit - 1) / nsplit * kPT;
@@ -77,19 +77,13 @@ inline PrePlan prefill_plan(int B, int Hq, int Hkv, int L, int S, int window, in
 struct PreLayout {
   size_t o, ml, total;
 };
-inline PreLayout prefill_layout(const PrePlan& pl, int D) {
+inline PreLayout prefill_layout(const PrePlan& pl, int D, bool f32_partials) {
   PreLayout l;
   const size_t slots = (size_t)pl.nunits * pl.nsplit * kPRows;
   l.o = kCounterBytes;
-  l.ml = l.o + slots * D * sizeof(uint16_t);  // fp16 rows
-  l.total = l.ml + (slots * 4 * sizeof(float) + 255) / 256 * 256;  // (m, l, 2^e, -) records
+  l.ml = l.o + slots * D * (f32_partials ? sizeof(float) : sizeof(uint16_t));
+  l.total = l.ml + (slots * 4 * sizeof(float) + 255) / 256 * 256;  // (m, l, the row's factor, -) records
   return l;
-}
-
-// The plan with as many splits as `bytes` of workspace hold (at 64 and 128 dims always all of them).
-inline PrePlan fit_plan(PrePlan pl, int D, size_t bytes) {
-  while (pl.nsplit > 1 && prefill_layout(pl, D).total > bytes) set_splits(&pl, pl.nsplit - 1);
-  return pl;
 }
 
 // Workgroup `wg` of the launch's `grid` = nbk rowblocks nsplit: its (sequence, KV head) pair, row block and

@@ -40,6 +40,41 @@ def test_splits(B, Hq, Hkv, L, S, D, bits, dtype, lens):
     assert torch.equal(out, kernels.attention(q, kt, vt, scale, kernel="prefill", **kw))
 
 
+@pytest.mark.parametrize("form,B,Hq,Hkv,L,S,D,bits", [
+    ("causal", 1, 2, 2, 100, 5000, 96, 8),    # many splits, merged by their own launch
+    ("causal", 1, 4, 4, 900, 900, 96, 4),     # a few, merged by the last of them
+    ("causal", 1, 8, 2, 100, 3000, 64, 16),
+    ("causal", 1, 8, 4, 900, 900, 64, 16),
+    ("masked", 1, 8, 2, 100, 5000, 128, 8),
+    ("masked", 1, 8, 2, 160, 3000, 64, 4),
+    ("masked", 1, 8, 2, 100, 5000, 128, 16),
+    ("masked", 2, 8, 4, 130, 700, 96, 8),
+])
+def test_partials_in_fp32(form, B, Hq, Hkv, L, S, D, bits):
+    """Zero queries over whole-number values: every probability and every sum is exact, so an output is the
+    correctly rounded mean but for the last bits of one fp32 division (a share of about 2^-12 near a tie).
+    Partial rows rounded to fp16 on the way would miss it in a quarter of the elements or so."""
+    print(f"fp32 partials {form} {B} {Hq} {Hkv} L={L} S={S} D={D} bits={bits}", flush=True)
+    G, top = (32 if D == 96 else 64), (255 if bits != 4 else 15)
+    v = torch.randint(0, top + 1, (B, Hkv, S, D), generator=torch.Generator().manual_seed(4700 + S + D))
+    v[..., ::32], v[..., 1::32] = 0, top  # the groups' extremes: scale -1, bias `top`
+    k = seeded_normal((B, Hkv, S, D), 4701, torch.float16, DEV)
+    vd = v.half().to(DEV)
+    kt, vt = (k, vd) if bits == 16 else (kernels.quantize(k, G, bits), kernels.quantize(vd, G, bits))
+    q = torch.zeros((B, Hq, L, D), dtype=torch.float16, device=DEV)
+    visible = torch.ones((L, S), dtype=torch.bool).tril(S - L)
+    if form == "masked":
+        visible[:, ::3] = False  # (no structure that the causal kernels take)
+        mask = visible.to(DEV)
+        out = kernels.masked_attention(q, kt, vt, 0.1, mask, group_size=G, bits=bits if bits != 16 else 8)
+    else:
+        out = kernels.attention(q, kt, vt, 0.1, causal=True, group_size=G, bits=bits if bits != 16 else 8, kernel="prefill")
+    mean = visible.double() @ v.double() / visible.double().sum(-1, keepdim=True)
+    want = mean.half().repeat_interleave(Hq // Hkv, dim=1)
+    off = (out.cpu() != want).double().mean().item()
+    assert off < 0.005, off
+
+
 def test_unquantized_d64_rows_of_8_bytes():
     """Unquantized head_dim-64 prefill into output rows that are only 8-byte aligned, many splits and none."""
     for L, S in ((100, 3000), (300, 300)):

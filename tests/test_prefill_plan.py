@@ -1,5 +1,5 @@
-"""The prefill kernel's host plan on the CPU (csrc/prefill_plan.h): whatever splits a workspace leaves a
-call, every (pair, row block, split) is served by exactly one workgroup. (A plan whose splits were cut
+"""The prefill kernel's host plan on the CPU (csrc/prefill_plan.h): whatever number of splits a call runs
+with, every (pair, row block, split) is served by exactly one workgroup. (A plan whose splits were cut
 after its numbering was chosen sent workgroups to row block -1.)"""
 
 import subprocess

@@ -51,6 +51,21 @@ def test_oracle_rule_is_the_smallest_exponent():
 
 
 @pytest.mark.parametrize("bits", [4, 8])
+def test_fp16_groups_at_both_ends_of_the_type_fit_fp16_operands(bits):
+    """The prefill kernels' operands hold s c + b in fp16. The quantizer rounds its zero point to a code q0 >=
+    2^(bits - 1) of the larger extreme b, so |b + n s| <= (n / q0 - 1) |b| stays below |b| by more than the
+    scale's own rounding moves it."""
+    rng = np.random.default_rng(17)
+    for G in (32, 64, 128):
+        for lo, hi in ((1.0, 1.0), (1.0, 0.999), (0.998, 1.0), (1.0, 0.9), (0.7, 1.0), (1.0, 0.5)):
+            x = rng.uniform(-65504.0 * lo, 65504.0 * hi, size=(256, G)).astype(np.float32)
+            x[:, 0], x[:, 1] = -65504.0 * lo, 65504.0 * hi
+            _, s, b = Q.quantize(Q.to_bits(x, "float16"), "float16", G, bits)
+            s, b = (Q.from_bits(t, "float16").astype(np.float64) for t in (s, b))
+            assert np.abs(b).max() <= 65504.0 and np.abs(b + (2**bits - 1) * s).max() <= 65504.0
+
+
+@pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_host_computation_matches_oracle(bits, dtype):
     rng = np.random.default_rng(11 + bits)
