@@ -10,7 +10,7 @@ size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int 
   size_t n = 256;
   for (int causal : {0, 1}) {
     const PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, window, causal);
-    // (the size serves quantized and unquantized calls: at 64 dims the latter's partials are fp32)
+    // (the size serves quantized and unquantized calls: at 64 dims the latter's partials are fp32, the larger)
     if (pl.nsplit > 1) n = std::max(n, prefill_layout(pl, D, D != 128).total);
   }
   return n;

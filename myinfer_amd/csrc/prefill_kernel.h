@@ -1148,24 +1148,33 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
     //    u (0 .. QW - 1) of 16 bytes at byte ((s * kPW + wave) * QW + u) * 1024 + 16 lane of the unit's o
     //    block; word u packs value groups 2u and 2u + 1 (group 4 db + c = oacc[db][4c .. 4c+3]).
     //    Record of row r at byte 16 (s * kPRows + r) of the unit's record block.
-    //  * With fp32 partials (kF32Partials) a row is o itself, word u (0 .. 2 QW - 1) value group u, and its
-    //    record (m, l, 2^E_V): the merge scales row s by w_s 2^E_V.
+    //  * With fp32 partials (kF32Partials) a row is o itself in the cache's units, word u (0 .. 2 QW - 1) value
+    //    group u, and its record (m, l), 8 bytes: the merge scales row s by w_s.
     constexpr bool F32P = kF32Partials<BITS, D, MASKED>;
     constexpr int NW = F32P ? 2 * QW : QW;       // 16-byte words of a lane's row
     constexpr uint32_t split_o = kPW * NW * 1024;
     const __amdgpu_buffer_rsrc_t ro =
         make_rsrc((const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * split_o, (uint32_t)p.nsplit * split_o);
-    const __amdgpu_buffer_rsrc_t rm = make_rsrc(p.part_ml + (int64_t)unit * p.nsplit * (kPRows * 4),
-                                                (uint32_t)p.nsplit * (kPRows * 16));
+    constexpr uint32_t REC = F32P ? 8 : 16;  // bytes of a record
+    const __amdgpu_buffer_rsrc_t rm = make_rsrc(p.part_ml + (int64_t)unit * p.nsplit * (kPRows * REC / 4),
+                                                (uint32_t)p.nsplit * (kPRows * REC));
     const uint32_t lo = (uint32_t)wave * (NW * 1024) + 16 * lane;
-    const uint32_t row_ml = 16 * (wave * 32 + qc);
+    const uint32_t row_ml = REC * (wave * 32 + qc);
+    auto load_rec = [&](int s) -> f4 {
+      if constexpr (F32P) {
+        const float2 r = load_agent_b64(rm, row_ml, s * (kPRows * REC));
+        return f4{r.x, r.y, 1.0f, 0.0f};
+      } else {
+        return load_agent_b128(rm, row_ml, s * (kPRows * REC));
+      }
+    };
     f4 own[NW];
-    float own_sc = vback;  // the V operands were staged times 2^-E_V
-    if constexpr (F32P) {
+    float own_sc = 1.0f;
+    if constexpr (F32P) {  // (the V operands were staged times 2^-E_V)
 #pragma unroll
       for (int g = 0; g < NW; ++g)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) own[g][i] = oacc[g >> 2][4 * (g & 3) + i];
+        for (int i = 0; i < 4; ++i) own[g][i] = oacc[g >> 2][4 * (g & 3) + i] * vback;
     } else {
       const float inv_l = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
       float mx = 0.0f;
@@ -1179,7 +1188,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
       int ex = 0;
       if (mx > 0.0f) frexpf(mx, &ex);
       const int e = mx > 0.0f ? min(max(ex - 14, -100), 100) : 0;
-      own_sc *= ldexpf(1.0f, e);
+      own_sc = ldexpf(1.0f, e) * vback;  // the V operands were staged times 2^-E_V
       const float f = ldexpf(inv_l, -e);
 #pragma unroll
       for (int u = 0; u < NW; ++u) {
@@ -1195,7 +1204,11 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
     }
 #pragma unroll
     for (int u = 0; u < NW; ++u) store_agent_b128(ro, lo + u * 1024 + split * split_o, own[u]);
-    if (hh == 0) store_agent_b128(rm, row_ml + split * (kPRows * 16), f4{m_run, l_tot, own_sc, 0.0f});
+    if constexpr (F32P) {
+      if (hh == 0) store_agent_b64(rm, row_ml + split * (kPRows * REC), make_float2(m_run, l_tot));
+    } else {
+      if (hh == 0) store_agent_b128(rm, row_ml + split * (kPRows * REC), f4{m_run, l_tot, own_sc, 0.0f});
+    }
     if (!p.fused) return;
     // The stores are acknowledged (written through to the device's coherence point) before the
     // arrival is counted, so the last arrival sees every split's partials.
@@ -1210,7 +1223,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
     float M = l_tot > 0.0f ? m_run : -INFINITY;
     for (int s2 = 0; s2 < nsplit; ++s2) {
       if (s2 == split) continue;
-      const f4 rec = load_agent_b128(rm, row_ml, s2 * (kPRows * 16));
+      const f4 rec = load_rec(s2);
       if (rec[1] > 0.0f) M = fmaxf(M, rec[0]);
     }
     // the splits are summed in split order, each term one explicit fma
@@ -1226,13 +1239,13 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
 #pragma unroll
         for (int u = 0; u < NW; ++u) po[u] = own[u];
       } else {
-        rec = load_agent_b128(rm, row_ml, s2 * (kPRows * 16));
+        rec = load_rec(s2);
 #pragma unroll
         for (int u = 0; u < NW; ++u) po[u] = load_agent_b128(ro, lo + u * 1024, s2 * split_o);
       }
       const float w = (M == -INFINITY || rec[1] <= 0.0f) ? 0.0f : exp2_fast(rec[0] - M);
       l_acc = fmaf(w, rec[1], l_acc);
-      const float F = F32P ? w * rec[2] : (w * rec[1]) * rec[2];
+      const float F = F32P ? w : (w * rec[1]) * rec[2];
 #pragma unroll
       for (int u = 0; u < NW; ++u) {
         if constexpr (F32P) {
@@ -1315,6 +1328,7 @@ template <typename T, int D, bool F32P, bool MASKED = false>
 __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) {
   constexpr int QW = F32P ? D / 8 : D / 16;  // words per row
   constexpr int NV = F32P ? 4 : 8;           // values per word
+  constexpr int NREC = F32P ? 2 : 4;         // floats per record
   constexpr int split_o = kPW * QW * 1024;
   __shared__ float s_m[kPW][64], s_l[kPW][64];
   __shared__ __align__(16) float s_o[kPW][64][NV];
@@ -1335,7 +1349,7 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
   }
   if (ks.nsplit == 1 || fr0 + 32 * w >= p.nrows) return;
   const uint8_t* po = (const uint8_t*)p.part_o + (int64_t)unit * p.nsplit * split_o + (w * QW + u) * 1024 + 16 * lane;
-  const f4* rec = (const f4*)(p.part_ml + (int64_t)unit * p.nsplit * (kPRows * 4)) + 32 * w + (lane & 31);
+  const float* rec = p.part_ml + (int64_t)unit * p.nsplit * (kPRows * NREC) + (32 * w + (lane & 31)) * NREC;
   constexpr int CH = 4;
   float M = -INFINITY, l = 0.0f, acc[NV] = {};
   for (int s0 = wave; s0 < ks.nsplit; s0 += kPW * CH) {
@@ -1344,7 +1358,12 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int s = min(s0 + kPW * i, ks.nsplit - 1);  // past the last split it is re-read, and not counted
-      r[i] = rec[s * kPRows];
+      if constexpr (F32P) {
+        const float2 x = *(const float2*)(rec + s * (kPRows * NREC));
+        r[i] = f4{x.x, x.y, 1.0f, 0.0f};
+      } else {
+        r[i] = *(const f4*)(rec + s * (kPRows * NREC));
+      }
       v[i] = *(const u4*)(po + (int64_t)s * split_o);
     }
     float Mn = M;
@@ -1362,7 +1381,7 @@ __global__ __launch_bounds__(kPW * 64) void prefill_combine_kernel(PreParams p) 
       // a row that saw no key in the split counts 0, but for NaN (a poisoned row block)
       const float ws = r[i][1] > 0.0f ? exp2_fast(r[i][0] - M) : 0.0f;
       l += ws * r[i][1];
-      const float F = (F32P ? ws : ws * r[i][1]) * r[i][2];
+      const float F = F32P ? ws : (ws * r[i][1]) * r[i][2];
 #pragma unroll
       for (int e = 0; e < NV; ++e) {
         const uint32_t x = v[i][F32P ? e : e >> 1];

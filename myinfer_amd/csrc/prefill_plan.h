@@ -82,7 +82,8 @@ inline PreLayout prefill_layout(const PrePlan& pl, int D, bool f32_partials) {
   const size_t slots = (size_t)pl.nunits * pl.nsplit * kPRows;
   l.o = kCounterBytes;
   l.ml = l.o + slots * D * (f32_partials ? sizeof(float) : sizeof(uint16_t));
-  l.total = l.ml + (slots * 4 * sizeof(float) + 255) / 256 * 256;  // (m, l, the row's factor, -) records
+  // records: (m, l), or (m, l, 2^e, -) of an fp16 row
+  l.total = l.ml + (slots * (f32_partials ? 2 : 4) * sizeof(float) + 255) / 256 * 256;
   return l;
 }
 
