@@ -18,7 +18,7 @@ size_t prefill_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int S, int 
 
 template <typename T, int BITS, bool PAGED = false, int G = 64, int D = 128>
 static hipError_t launch_prefill_t(const PreParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL((prefill_attn_kernel<T, BITS, PAGED, G, D>), dim3(p.nunits * p.nsplit), dim3(kPW * 64), 0, stream,
+  hipLaunchKernelGGL((prefill_attn_kernel<T, BITS, PAGED, G, D>), dim3(prefill_grid(p)), dim3(kPW * 64), 0, stream,
                      p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.nsplit == 1 || p.fused) return e;
@@ -83,10 +83,11 @@ static PreParams prefill_params(const kvq_rows* q, const int32_t* seq_lens, cons
   p.rowblocks = pl.rowblocks;
   p.nsplit = pl.nsplit;
   p.chunk = pl.chunk;
-  p.longest_first = pl.longest_first;
+  p.order = pl.order;
+  p.nbk = pl.nbk;
+  p.lo = pl.lo;
   p.fused = pl.nsplit <= kPFusedMaxSplit;
   p.nunits = pl.nunits;
-  p.xcd_remap = ((int64_t)pl.nunits * pl.nsplit) % kXcds == 0;
   p.scale_log2 = scale * 1.4426950408889634f;
   p.causal = causal;
   p.window = window;
@@ -175,8 +176,7 @@ struct MaskedPlan {
 };
 static bool plan_masked(int B, int Hq, int Hkv, int L, int D, int S, const kvq_mask* mask, size_t bytes, MaskedPlan* m) {
   PrePlan pl = prefill_plan(B, Hq, Hkv, L, S, 0, 0);
-  pl.unequal = true;  // most masks are causal and then some: the row blocks of the last positions first
-  set_splits(&pl, pl.nsplit);
+  pl.order = kMasked;  // most masks are causal and then some: the row blocks of the last positions first
   m->nwords = ((S + kPT - 1) / kPT + 63) / 64;
   const size_t need = (size_t)B * (mask->stride_kvh ? Hkv : 1) * pl.rowblocks * m->nwords * 16;
   for (;; set_splits(&pl, pl.nsplit - 1)) {

@@ -28,8 +28,8 @@
 //    the fp16 operands: the row blocks that read one return NaN rather than wrong finite values.
 //  * Online softmax with threshold rescaling (a row's running maximum moves only when a tile's
 //    maximum exceeds it by more than 2^6), fp32 accumulators.
-//  * Long key ranges are split over several workgroups; the last split of a row block to finish
-//    merges the (m, l, o) partials of the others (log-sum-exp) and writes the output.
+//  * Long key ranges are split over several workgroups. Up to 4 splits of a row block are merged (log-sum-exp
+//    over their (m, l, o) partials) by the last of them to finish, more by a launch of their own.
 //  * An unquantized fp16/bf16 cache (BITS == 16, head_dim 128 or 64) takes a simpler loop: K operands
 //    straight from the raw ring, only V^T staged, the MFMAs in the cache's type.
 
@@ -147,9 +147,7 @@ struct PreParams {
   float* part_o;
   float* part_ml;
   unsigned* counters;  // arrivals per unit, zero between launches
-  int xcd_remap;       // 1: the grid is a multiple of the XCD count (see prefill_wg)
-  int longest_first;   // row blocks of unequal length, numbered from the longest down: 1 over all (sequence,
-                       // KV head) pairs of an XCD, 2 within each pair (set_splits)
+  int order, nbk, lo;  // how workgroups are numbered (prefill_wg)
   int Hq, Hkv, L, S, rep, nrows, rowblocks, nsplit, nunits;
   int chunk;           // keys per split (a multiple of 64); see split_keys
   int fused;           // 1: the last split of a row block merges; 0: prefill_combine_kernel does
@@ -198,23 +196,6 @@ __device__ __forceinline__ MaskSplit split_masked(const PreParams& p, int b, int
   m.chunk = max(p.chunk / kPT, (m.n + p.nsplit - 1) / p.nsplit);
   m.nsplit = max((m.n + m.chunk - 1) / m.chunk, 1);
   return m;
-}
-
-// The keys the rows [fr0, frl] of a row block see, in whole tiles ([lo, hi), lo rounded down to a
-// tile), and the splits they are cut into: `chunk` keys each, so that workgroups of long and short
-// row blocks (a causal prompt's last and first) are about as long, the short ones taking fewer.
-struct KeySplit {
-  int lo, hi, chunk, nsplit;
-};
-__device__ __forceinline__ KeySplit split_keys(const PreParams& p, int S_b, int fr0, int frl) {
-  const int pos_min = S_b - p.L + fr0 / p.rep, pos_max = S_b - p.L + frl / p.rep;
-  KeySplit k;
-  k.hi = p.causal ? min(S_b, pos_max + 1) : S_b;
-  k.lo = (p.window > 0 ? max(0, pos_min - p.window + 1) : 0) & ~(kPT - 1);
-  const int span = max(k.hi - k.lo, 0);
-  k.chunk = max(p.chunk, ((span + p.nsplit - 1) / p.nsplit + kPT - 1) / kPT * kPT);
-  k.nsplit = max((span + k.chunk - 1) / k.chunk, 1);
-  return k;
 }
 
 // V^T slot of key `kk` (0..63) inside a tile: the 16 keys of PV k-step j = kk / 16 are stored so
@@ -532,7 +513,7 @@ __global__ __launch_bounds__(kPW * 64, 1) void prefill_attn_kernel(PreParams p) 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qc = lane & 31, hh = lane >> 5;
 
-  const PreWg wg = prefill_wg((int)blockIdx.x, (int)gridDim.x, p.rowblocks, p.nsplit, p.xcd_remap, p.longest_first);
+  const PreWg wg = prefill_wg(p, (int)blockIdx.x, (int)gridDim.x);
   const int rb = wg.rb, split = wg.split, bk = wg.bk;  // bk = b * Hkv + kvh
   const int b = bk / p.Hkv, kvh = bk % p.Hkv;
   const int unit = bk * p.rowblocks + rb;

@@ -80,7 +80,8 @@ __global__ __launch_bounds__(kClassWaves * 64) void mask_classes_kernel(PreParam
       }
 #pragma unroll
       for (int c = 0; c < CH; ++c) {
-        // hidden: the value in log2 units is -inf (a type's lowest value times log2 e is, in fp32)
+        // hidden: the value in log2 units is -inf (as the lowest value of fp32 and bf16 times log2 e is in fp32;
+        // fp16's is -94502, a finite addend, whose tiles are computed)
         const float a = EL == 4 ? __uint_as_float(x[c])
                                 : p.mask_kind == KVQ_MASK_BF16 ? to_float((uint16_t)x[c], BF16{}) : to_float((uint16_t)x[c], F16{});
         any |= !(a * 1.4426950408889634f == -INFINITY);
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(kClassWaves * 64) void mask_classes_kernel(PreParam
 
 template <typename T, int BITS, int G, int D>
 static hipError_t launch_t(const PreParams& p, hipStream_t stream) {
-  const dim3 grid(p.nunits * p.nsplit), block(kPW * 64);
+  const dim3 grid(prefill_grid(p)), block(kPW * 64);
   if (p.mask_kind == KVQ_MASK_BOOL) {
     hipLaunchKernelGGL((prefill_attn_kernel<T, BITS, false, G, D, 1>), grid, block, 0, stream, p);
   } else if constexpr (BITS == 16) {

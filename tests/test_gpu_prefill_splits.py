@@ -17,14 +17,16 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,L,S,D,bits,dtype,lens", [
-    (1, 8, 8, 1100, 1100, 128, 8, torch.float16, None),          # a pair per XCD, 5 row blocks, 4 splits
-    (1, 8, 2, 520, 520, 128, 4, torch.bfloat16, None),           # a pair's row blocks over 4 XCDs
-    (3, 4, 1, 700, 700, 64, 8, torch.float16, [700, 701 - 64, 700 - 250]),  # 3 pairs: numbered within each
+    (1, 8, 8, 1100, 1100, 128, 8, torch.float16, None),          # a pair per XCD, 5 row blocks of 1 to 4 splits
+    (1, 8, 2, 520, 520, 128, 4, torch.bfloat16, None),           # 2 pairs
+    (3, 4, 1, 700, 700, 64, 8, torch.float16, [700, 701 - 64, 700 - 250]),  # 3 pairs
     (1, 16, 16, 900, 900, 64, 8, torch.float16, None),           # two pairs per XCD
     (1, 4, 2, 70, 4096, 128, 8, torch.float16, None),            # 16 splits, a ragged row block
     (2, 2, 1, 300, 9000, 64, 4, torch.bfloat16, [9000, 310]),    # 64 splits for one sequence, two for the other
     (1, 8, 1, 40, 16500, 128, 8, torch.float16, None),           # 65 splits: more than one round of the merge
     (1, 2, 2, 100, 5000, 96, 8, torch.float16, None),
+    (1, 2, 2, 1600, 1600, 128, 8, torch.float16, None),          # a prompt of 5 splits: a merge launch over 1 to 5
+    (2, 1, 1, 1500, 1500, 64, 4, torch.float16, [1500, 700]),    # 6
 ])
 def test_splits(B, Hq, Hkv, L, S, D, bits, dtype, lens):
     G = 32 if D == 96 else 64

@@ -1,6 +1,7 @@
 """The prefill kernel's host plan on the CPU (csrc/prefill_plan.h): whatever number of splits a call runs
-with, every (pair, row block, split) is served by exactly one workgroup. (A plan whose splits were cut
-after its numbering was chosen sent workgroups to row block -1.)"""
+with, every (pair, row block, split) that holds keys is served by exactly one workgroup, and the XCDs get
+equal shares of a causal prompt. (A plan whose splits were cut after its numbering was chosen sent workgroups
+to row block -1; one that dealt row blocks and splits to the XCDs in turn gave some the empty splits only.)"""
 
 import subprocess
 from pathlib import Path
