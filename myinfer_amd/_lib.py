@@ -263,6 +263,11 @@ class AppendState(ctypes.Structure):
                 ("group", ctypes.c_int32), ("code", ctypes.c_int32), ("device", ctypes.c_int32), ("stream", c_void_p)]
 
 
+def bind_host(module, *addresses: int) -> None:
+    """Give the host path the library's entry points: decode, prefill and their workspace sizes."""
+    module.bind(*addresses)
+
+
 _host = None
 
 
@@ -277,7 +282,7 @@ def host():
             raise ImportError(f"_kvqhost.so does not load ({e}): build it with `python -m myinfer_amd._build`") from e
         with _lock:
             if _host is None:
-                _kvqhost.bind(*(ctypes.cast(fn, c_void_p).value for fn in (
+                bind_host(_kvqhost, *(ctypes.cast(fn, c_void_p).value for fn in (
                     handle.kvq_decode_attn, handle.kvq_prefill_attn, handle.kvq_decode_workspace_size,
                     handle.kvq_prefill_workspace_size)))
                 _host = _kvqhost

@@ -5,7 +5,9 @@
 // In Python the two calls of a decode step cost about 45 us of host time, three times their kernels' time
 // on a 4096-token cache of 8 heads; here about 10. Every function returns None for anything but those
 // forms (other types, devices, strides, a call the library refuses): the Python path then serves the call
-// or raises, so that what is accepted and what is refused has one definition.
+// or raises, so that what is accepted and what is refused has one definition. A launch that failed is not
+// tried again: the Python side gets its (negative) status to raise. The interpreter lock is released
+// around the library's calls, which may wait for room in a full queue.
 
 #include <ATen/ATen.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -38,6 +40,18 @@ struct AppendState {
 };
 
 PyObject* none() { Py_RETURN_NONE; }
+
+// What a library call that did not return KVQ_OK becomes: see above. (Nothing was launched by a refused one.)
+PyObject* failed(int rc) {
+  if (rc == KVQ_ERR_HIP) return PyLong_FromLong(rc);
+  return none();
+}
+
+// Releases the interpreter lock while it lives.
+struct Unlocked {
+  PyThreadState* st = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(st); }
+};
 
 int dtype_code(at::ScalarType t) {
   return t == at::kHalf ? KVQ_DTYPE_F16 : t == at::kBFloat16 ? KVQ_DTYPE_BF16 : -1;
@@ -80,7 +94,8 @@ bool qtensor_of(const Triple& t, int64_t B, int64_t Hkv, int64_t S, int64_t D, i
 }
 
 // attention(queries, keys, values, scale, causal, window, seq_lens, group_size, bits, prefill, k_range, v_range,
-//           workspace, stream) -> the output, the workspace bytes needed if the given ones are too few, or None
+//           workspace, stream) -> the output, the workspace bytes needed if the given ones are too few, the negative
+//           status of a failed launch, or None
 PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 14 || !g.decode || !THPVariable_Check(a[0])) return none();
   try {
@@ -124,17 +139,23 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (ws.nbytes() < need) return PyLong_FromSize_t(need);
     at::Tensor out = at::empty({B, Hq, L, D}, q.options().requires_grad(false));
     const kvq_rows orr = {out.data_ptr(), Hq * L * D, L * D, D};
-    const int rc = (prefill ? g.prefill : g.decode)(&qr, &kq, &vq, lens, &orr, (int)B, (int)Hq, (int)Hkv, (int)L, (int)D,
-                                                    (int)S, (int)bits, (int)group, code, (float)scale, (int)causal,
-                                                    (int)window, ws.data_ptr(), ws.nbytes(), stream);
-    if (rc != KVQ_OK) return none();
+    void* const wp = ws.data_ptr();
+    const size_t wn = ws.nbytes();
+    int rc;
+    {
+      Unlocked u;
+      rc = (prefill ? g.prefill : g.decode)(&qr, &kq, &vq, lens, &orr, (int)B, (int)Hq, (int)Hkv, (int)L, (int)D, (int)S,
+                                            (int)bits, (int)group, code, (float)scale, (int)causal, (int)window, wp, wn,
+                                            stream);
+    }
+    if (rc != KVQ_OK) return failed(rc);
     return THPVariable_Wrap(std::move(out));
   } catch (...) {
     return none();
   }
 }
 
-// append(state address, keys, values, row_offset, rope_offset) -> True, or None
+// append(state address, keys, values, row_offset, rope_offset) -> True, the negative status of a failed launch, or None
 PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 5 || !THPVariable_Check(a[1]) || !THPVariable_Check(a[2])) return none();
   try {
@@ -153,16 +174,19 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (k.size(0) != st->B || k.size(1) != st->H || row < 0 || row + L > st->rows || L > INT32_MAX) return none();
     if (D * st->bits / 32 != st->code_words || D / st->group != st->groups) return none();
     int rc;
-    if (st->rope) {
-      kvq_rope_params rp = *st->rope;
-      rp.offset = pos;
-      rc = ((RopeAppendFn)st->fn)(&kr, st->kq, &vr, st->vq, &rp, row, (int)st->B, (int)st->H, (int)L, (int)D, st->bits,
-                                  st->group, st->code, st->stream);
-    } else {
-      rc = ((AppendFn)st->fn)(&kr, st->kq, &vr, st->vq, row, (int)st->B, (int)st->H, (int)L, (int)D, st->bits, st->group,
-                              st->code, st->stream);
+    {
+      Unlocked u;
+      if (st->rope) {
+        kvq_rope_params rp = *st->rope;
+        rp.offset = pos;
+        rc = ((RopeAppendFn)st->fn)(&kr, st->kq, &vr, st->vq, &rp, row, (int)st->B, (int)st->H, (int)L, (int)D, st->bits,
+                                    st->group, st->code, st->stream);
+      } else {
+        rc = ((AppendFn)st->fn)(&kr, st->kq, &vr, st->vq, row, (int)st->B, (int)st->H, (int)L, (int)D, st->bits, st->group,
+                                st->code, st->stream);
+      }
     }
-    if (rc != KVQ_OK) return none();
+    if (rc != KVQ_OK) return failed(rc);
     Py_RETURN_TRUE;
   } catch (...) {
     return none();

@@ -216,6 +216,7 @@ class AppendCall:
         lib = _lib.lib()
         self._fn = lib.kvq_rope_quantize_append if rope is not None else lib.kvq_quantize_append
         self._stream = _lib.stream_ptr(self._dev)
+        self._symbol = "kvq_rope_quantize_append" if rope is not None else "kvq_quantize_append"
         self._host = _lib.host().append
         self._state = _lib.AppendState(
             ctypes.cast(self._fn, ctypes.c_void_p).value, ctypes.addressof(self._kq),
@@ -227,8 +228,11 @@ class AppendCall:
     def __call__(self, k: torch.Tensor, v: Optional[torch.Tensor], row_offset: int,
                  rope_offset: Optional[int] = None) -> None:
         # the native host path; anything it does not take is checked, served or refused below
-        if self._host(self._state_ptr, k, v, row_offset, row_offset if rope_offset is None else rope_offset):
+        done = self._host(self._state_ptr, k, v, row_offset, row_offset if rope_offset is None else rope_offset)
+        if done is True:
             return
+        if done is not None:  # a failed launch, which is not tried again
+            _lib.check(done, self._symbol)
         if k.dtype != self._dtype or k.device != self._dev or k.dim() != 4 or k.stride(-1) != 1:
             raise ValueError("rows must match the prepared dtype and device, as [B, H, L, D] with D contiguous")
         B, H, L, D = k.shape
@@ -257,7 +261,7 @@ class AppendCall:
             rc = self._fn(ctypes.byref(kr), ctypes.byref(self._kq), vr_p, vq_p, ctypes.byref(self._rp),
                           int(row_offset), B, H, L, D, self._bits, self._group, self._code, self._stream)
         if rc:
-            _lib.check(rc, "kvq_rope_quantize_append" if self._rp is not None else "kvq_quantize_append")
+            _lib.check(rc, self._symbol)
 
 
 def prepare_append(k_dst: Triple, v_dst: Optional[Triple] = None, *, group_size: int = 64, bits: int = 8,
@@ -533,8 +537,10 @@ def layer_attention(queries: torch.Tensor, keys, values, scale: float, *, causal
             0 if kw is None else kw.data_ptr(), 0 if vw is None else vw.data_ptr())
     call = _lib.host().attention
     out = call(*args, ws, stream)
-    if type(out) is int:  # the bytes of workspace it needs
+    if type(out) is int and out > 0:  # the bytes of workspace it needs
         out = call(*args, _workspace(queries.device, stream, out), stream)
+    if type(out) is int:  # a failed launch, which is not tried again
+        _lib.check(out, "kvq_prefill_attn" if prefill else "kvq_decode_attn")
     return out
 
 

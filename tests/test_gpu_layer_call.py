@@ -1,9 +1,14 @@
 """The native host path of a layer's step (csrc/host): the same results, bit for bit, as the prepared calls
 it stands for, over the forms it takes, and the same errors for the forms it hands back."""
 
+import ctypes
+import subprocess
+import threading
+
 import pytest
 import torch
 
+from myinfer_amd import _lib
 from myinfer_amd import attention as A
 from myinfer_amd import kernels
 from myinfer_amd.cache import QuantizedKVCache
@@ -91,3 +96,59 @@ def test_append_forms_and_streams():
         for a, b in zip(got[0] + got[1], ref.keys + ref.values):
             assert a.shape[2] == 9 and a.stride() == b.stride()
             assert torch.equal(a.view(torch.int16), b[:, :, :9].view(torch.int16))
+
+
+STUBS = """
+#include <unistd.h>
+extern "C" {
+volatile int go = 0, calls = 0, late = 0;
+int waits() {  // until `go` is set, at most 3 s
+  for (int i = 0; i < 3000 && !go; ++i) usleep(1000);
+  late = !go;
+  return 0;
+}
+int fails() { return ++calls, -4; }  // KVQ_ERR_HIP
+size_t bytes() { return 256; }
+}
+"""
+
+
+@pytest.fixture
+def stubs(tmp_path):
+    (tmp_path / "stubs.cpp").write_text(STUBS)
+    subprocess.run(["g++", "-shared", "-fPIC", str(tmp_path / "stubs.cpp"), "-o", str(tmp_path / "stubs.so")], check=True)
+    lib = ctypes.CDLL(str(tmp_path / "stubs.so"))
+    lib.addr = lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+    lib.get = lambda name: ctypes.c_int.in_dll(lib, name)
+    return lib
+
+
+def test_other_threads_run_during_a_call(stubs):
+    """A launch that waits (a full queue) does not hold the interpreter lock: here it waits for another thread."""
+    kt, vt = make_cache(1, 2, 64, 128, 8, torch.float16, 5600)
+    k = seeded_normal((1, 2, 1, 128), 5601, torch.float16, DEV)
+    call = kernels.prepare_append(kt, vt)
+    call._state.fn = stubs.addr("waits")
+    threading.Timer(0.05, lambda: setattr(stubs.get("go"), "value", 1)).start()
+    call(k, k, 0)
+    assert stubs.get("late").value == 0
+
+
+def test_a_failed_launch_raises_and_is_not_tried_again(stubs):
+    kt, vt = make_cache(1, 2, 64, 128, 8, torch.float16, 5700)
+    k = seeded_normal((1, 2, 1, 128), 5701, torch.float16, DEV)
+    call = kernels.prepare_append(kt, vt)
+    call._state.fn = stubs.addr("fails")
+    with pytest.raises(RuntimeError, match="status -4"):
+        call(k, k, 0)
+    assert stubs.get("calls").value == 1
+    h = _lib.host()
+    try:
+        _lib.bind_host(h, *(stubs.addr(n) for n in ("fails", "fails", "bytes", "bytes")))
+        with pytest.raises(RuntimeError, match="status -4"):
+            A.blocked_quantized_sdpa(k, kt, vt, 0.1, None)
+    finally:
+        _lib._host = None
+        _lib.host()
+    assert stubs.get("calls").value == 2
+    A.blocked_quantized_sdpa(k, kt, vt, 0.1, None)
