@@ -92,8 +92,8 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     tlib = _torch_lib_dir()
     host_tmp = HOST.with_suffix(".so.tmp")
     tinc = tlib.parent / "include"
-    host_cmd = ["g++", *HOST_FLAGS, "-shared", "-w", f"-I{tinc}", f"-I{tinc}/torch/csrc/api/include",
-                f"-I{sysconfig.get_paths()['include']}", str(CSRC / "host" / "host.cpp"), "-o", str(host_tmp), f"-L{tlib}",
+    host_cmd = ["g++", *HOST_FLAGS, "-shared", "-isystem", str(tinc), "-isystem", str(tinc / "torch/csrc/api/include"),
+                "-isystem", sysconfig.get_paths()["include"], str(CSRC / "host" / "host.cpp"), "-o", str(host_tmp), f"-L{tlib}",
                 "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{tlib}"]
     jobs = jobs or min(len(sources) + len(host_sources) + 1, max(1, os.cpu_count() or 1), 8)
     with cf.ThreadPoolExecutor(jobs) as ex:

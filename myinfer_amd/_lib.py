@@ -264,11 +264,17 @@ class AppendState(ctypes.Structure):
 
 
 def bind_host(module, *addresses: int) -> None:
-    """Give the host path the library's entry points: decode, prefill and their workspace sizes."""
-    module.bind(*addresses)
+    """Give the host path the library's entry points: decode, prefill and their workspace sizes. Raises
+    ImportError where it was built for another library, AppendState or torch."""
+    module.bind(*addresses, ABI_VERSION, ctypes.sizeof(AppendState), torch.__version__)
 
 
 _host = None
+
+
+def loaded_host():
+    """The native host path if a call has loaded it, else None."""
+    return _host
 
 
 def host():

@@ -323,7 +323,8 @@ class QuantizedKVCache:
     def fetch(self):
         """The (codes, scales, biases) views of the first `offset` rows, for K and for V."""
         o = self.offset
-        both = _lib.host().views(self.keys, self.values, o)
+        host = _lib.loaded_host()  # (an append has loaded it; views of a restored cache need no library)
+        both = host.views(self.keys, self.values, o) if host is not None else None
         if both is not None:
             return both
         return tuple(x[..., :o, :] for x in self.keys), tuple(x[..., :o, :] for x in self.values)

@@ -10,7 +10,9 @@
 // around the library's calls, which may wait for room in a full queue.
 
 #include <ATen/ATen.h>
+#include <string.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "../../../include/kvq.h"
 
@@ -223,10 +225,23 @@ PyObject* views(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
 }
 
-// bind(decode, prefill, decode_workspace_size, prefill_workspace_size): the library's entry points
+// bind(decode, prefill, decode_workspace_size, prefill_workspace_size, abi, state_bytes, torch): the library's
+// entry points; raises where this module was built against another ABI, AppendState or torch.
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 4) {
-    PyErr_SetString(PyExc_TypeError, "bind takes 4 addresses");
+  if (n != 7) {
+    PyErr_SetString(PyExc_TypeError, "bind takes 4 addresses, the ABI version, AppendState's size and torch's version");
+    return nullptr;
+  }
+  const long abi = PyLong_AsLong(a[4]), state = PyLong_AsLong(a[5]);
+  const char* torch = PyUnicode_AsUTF8(a[6]);
+  if (PyErr_Occurred() || !torch) return nullptr;
+  const size_t m = strlen(TORCH_VERSION);
+  if (abi != KVQ_ABI_VERSION || state != (long)sizeof(AppendState) || strncmp(torch, TORCH_VERSION, m) ||
+      (torch[m] >= '0' && torch[m] <= '9')) {
+    PyErr_Format(PyExc_ImportError,
+                 "_kvqhost.so was built for ABI version %d, an AppendState of %zu bytes and torch %s; here they are %ld, %ld "
+                 "and %s: rebuild it",
+                 KVQ_ABI_VERSION, sizeof(AppendState), TORCH_VERSION, abi, state, torch);
     return nullptr;
   }
   g.decode = (AttnFn)PyLong_AsVoidPtr(a[0]);

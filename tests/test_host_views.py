@@ -1,8 +1,10 @@
 """The native path's cache views on the CPU: the slices Python would take, and what it hands back."""
 
+import pytest
 import torch
 
 from myinfer_amd import _lib
+from myinfer_amd.cache import QuantizedKVCache
 
 
 def test_views_are_slices():
@@ -27,3 +29,31 @@ def test_handed_back():
     assert h.views(tr, tr, 5) is None and h.views(tr, tr, -1) is None
     assert h.attention(tr[0], tr, tr, 0.1, 0, 0, None, 64, 8, 0, 0, 0, None, 0) is None  # CPU tensors
     assert h.append(0, tr[0], tr[0], 0, 0) is None
+
+
+def test_another_build_is_refused(monkeypatch):
+    h = _lib.host()
+    for name, value in (("ABI_VERSION", _lib.ABI_VERSION + 1), ("AppendState", _lib.Rows)):
+        with monkeypatch.context() as m:
+            m.setattr(_lib, name, value)
+            with pytest.raises(ImportError, match="rebuild"):
+                _lib.bind_host(h, 0, 0, 0, 0)
+    for version in ("2.1.0", "", torch.__version__.split("+")[0] + "1"):
+        with monkeypatch.context() as m:
+            m.setattr(torch, "__version__", version)
+            with pytest.raises(ImportError, match="rebuild"):
+                _lib.bind_host(h, 0, 0, 0, 0)
+    assert _lib.lib() and h.attention(None) is None  # (bound as before)
+
+
+def test_views_of_a_restored_cache_need_no_library(monkeypatch):
+    def missing(*_):
+        raise ImportError("no library")
+
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setattr(_lib, "lib", missing)
+    c = QuantizedKVCache(group_size=64, bits=8)
+    c.keys = c.values = tuple(torch.arange(2 * 8 * w).view(1, 2, 8, w) for w in (4, 2, 2))
+    c.offset = 5
+    for tr in c.fetch():
+        assert all(torch.equal(a, b[..., :5, :]) for a, b in zip(tr, c.keys))
