@@ -224,6 +224,12 @@ int kvq_decode_attn_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qt
                            void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * 1 if kvq_decode_attn_masked may take the prefill kernel at these sizes (it then reads a bf16 cache's range
+ * words, and stays on the decode kernel without them), else 0. No counterpart in the reference.
+ */
+int kvq_masked_on_prefill(int B, int Hq, int Hkv, int L, int D, int S);
+
+/*
  * The same over an unquantized cache (kvq_decode_attn_dense's arguments and head dims; the prefill kernel
  * takes boolean and additive masks there, at head_dim 64 and 128).
  * Replaces the mask handling of mx.fast.scaled_dot_product_attention for array masks.

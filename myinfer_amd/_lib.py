@@ -136,6 +136,7 @@ SIGNATURES = {
     "kvq_decode_attn": (c_int, _ATTN_ARGS),
     "kvq_decode_attn_static": (c_int, _ATTN_ARGS[:-3] + [c_void_p]),  # no workspace: the library's scratch
     "kvq_decode_attn_masked": (c_int, _MASKED_ARGS),
+    "kvq_masked_on_prefill": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "kvq_decode_attn_dense_masked": (c_int, _DENSE_MASKED_ARGS),
     "kvq_paged_quantize_append": (
         c_int,

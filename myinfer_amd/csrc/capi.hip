@@ -560,6 +560,11 @@ static bool masked_on_prefill(const kvq_qtensor* k, const kvq_qtensor* v, const 
   return kvq::prefill_masked_fits(B, Hq, Hkv, L, D, S, mask, ws_bytes);
 }
 
+int kvq_masked_on_prefill(int B, int Hq, int Hkv, int L, int D, int S) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || S <= 0 || Hq % Hkv) return 0;
+  return kvq::prefill_masked_rows(B, Hq, Hkv, L, D, S) ? 1 : 0;
+}
+
 int kvq_decode_attn_masked(const kvq_rows* q, const kvq_qtensor* k, const kvq_qtensor* v, const kvq_rows* out, int B,
                            int Hq, int Hkv, int L, int D, int S, int bits, int group_size, int dtype, float scale,
                            const kvq_mask* mask, void* workspace, size_t workspace_bytes, void* stream) {
@@ -581,14 +586,13 @@ int kvq_decode_attn_dense_masked(const kvq_rows* q, const kvq_rows* k, const kvq
                                  int Hq, int Hkv, int L, int D, int S, int dtype, float scale, const kvq_mask* mask,
                                  void* workspace, size_t workspace_bytes, void* stream) {
   if (check_head_dim(D, "masked unquantized attention")) return KVQ_ERR_UNSUPPORTED;
-  int rc = check_attn_dense(q, k, v, out, B, Hq, Hkv, L, D, S, dtype, scale, 0,
-                            kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0), workspace, workspace_bytes);
+  const size_t ws = kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0);
+  int rc = check_attn_dense(q, k, v, out, B, Hq, Hkv, L, D, S, dtype, scale, 0, ws, workspace, workspace_bytes);
   if (rc || (rc = check_mask(mask))) return rc;
   if (D > 128)  // unquantized rows past 128 dims run through the head_dim-256 kernel
     return hip_status(kvq::launch_wide_dense(q, k, v, nullptr, out, B, Hq, Hkv, L, D, S, dtype, scale, 0, 0, workspace,
                                              (hipStream_t)stream, mask),
                       "decode_attn_dense_masked launch (the head_dim-256 kernel)");
-  const size_t ws = kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0);
   if (masked_on_prefill(nullptr, nullptr, out, B, Hq, Hkv, L, D, S, 64, dtype, mask, ws))
     return hip_status(kvq::launch_prefill_masked(q, nullptr, nullptr, k, v, out, B, Hq, Hkv, L, D, S, 16, 64, dtype, scale,
                                                  mask, workspace, ws, (hipStream_t)stream),

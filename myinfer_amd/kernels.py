@@ -8,6 +8,7 @@ zero-filled torch allocation cached per (device, stream); the library itself all
 from __future__ import annotations
 
 import ctypes
+import functools
 import weakref
 from dataclasses import dataclass
 from typing import Optional, Sequence, Tuple
@@ -602,6 +603,12 @@ def mask_view(mask: torch.Tensor, B: int, Hq: int, Hkv: int, L: int, S: int, lay
     return m5, (sb, skv, srep, sl)
 
 
+@functools.lru_cache(maxsize=256)
+def _masked_on_prefill(*sizes: int) -> int:
+    """kvq_masked_on_prefill, which follows from the sizes alone (a layer's foreign call costs 0.5 us)."""
+    return _lib.lib().kvq_masked_on_prefill(*sizes)
+
+
 def masked_attention(queries: torch.Tensor, keys, values, scale: float, mask: torch.Tensor, *, layout: str = "heads",
                      group_size: int = 64, bits: int = 8, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """softmax(scale * q K^T + mask) V under a general mask (boolean: visible keys; float: added to
@@ -640,28 +647,34 @@ def masked_attention(queries: torch.Tensor, keys, values, scale: float, mask: to
         queries = queries.contiguous()
     out = _check_out(out, queries, dev)
     lib = _lib.lib()
-    nbytes = lib.kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0)
-    if nbytes == 0:
-        raise NotImplementedError(f"decode attention does not support B={B} Hq={Hq} Hkv={Hkv} L={L} D={D} S={S}")
     stream = _lib.stream_ptr(dev)
-    ws = _workspace(dev, stream, nbytes)
     qr, orr = _lib.rows(queries), _lib.rows(out)
-    tail = (float(scale), ctypes.byref(desc), ws.data_ptr(), ws.numel() * ws.element_size(), stream)
     if dense:
+        symbol, fn = "kvq_decode_attn_dense_masked", lib.kvq_decode_attn_dense_masked
         kr, vr = _lib.rows(keys), _lib.rows(values)
-        rc = lib.kvq_decode_attn_dense_masked(ctypes.byref(qr), ctypes.byref(kr), ctypes.byref(vr), ctypes.byref(orr),
-                                              B, Hq, Hkv, L, D, S, _lib.dtype_code(queries.dtype), *tail)
-        _lib.check(rc, "kvq_decode_attn_dense_masked")
+        sizes = (B, Hq, Hkv, L, D, S, _lib.dtype_code(queries.dtype))
     else:
-        # a bf16 cache's range words, which only the prefill kernel reads; without them a call stays on the
-        # decode kernel, so finding them (3 us) waits for the sizes past which the library takes the other
-        passes = -(-(Hq // Hkv * L) // (4 if D == 96 else max(1, 1024 // D)))
-        words = queries.dtype == torch.bfloat16 and passes * B * Hkv * S >= 400_000
-        kq = _lib.qtensor(*keys, range_exp=range_word(keys[0]) if words else None)
-        vq = _lib.qtensor(*values, range_exp=range_word(values[0]) if words else None)
-        rc = lib.kvq_decode_attn_masked(ctypes.byref(qr), ctypes.byref(kq), ctypes.byref(vq), ctypes.byref(orr), B, Hq,
-                                        Hkv, L, D, S, int(bits), int(group_size), _lib.dtype_code(queries.dtype), *tail)
-        _lib.check(rc, "kvq_decode_attn_masked")
+        symbol, fn = "kvq_decode_attn_masked", lib.kvq_decode_attn_masked
+        kw = vw = None
+        # a bf16 cache's range words, which only the prefill kernel reads
+        if queries.dtype == torch.bfloat16 and _masked_on_prefill(B, Hq, Hkv, L, D, S):
+            kw, vw = range_word(keys[0]), range_word(values[0])
+        kr, vr = _lib.qtensor(*keys, range_exp=kw), _lib.qtensor(*values, range_exp=vw)
+        sizes = (B, Hq, Hkv, L, D, S, int(bits), int(group_size), _lib.dtype_code(queries.dtype))
+    args = (ctypes.byref(qr), ctypes.byref(kr), ctypes.byref(vr), ctypes.byref(orr), *sizes, float(scale), ctypes.byref(desc))
+    # the stream's workspace as it is: the library plans the call anyway and says if it is too small (asking
+    # first costs 1 us of the 8 to 10 us that a short call takes on the device)
+    ws = _workspaces.get((dev.index, stream))
+    rc = _lib.ERR_WORKSPACE if ws is None else fn(*args, ws.data_ptr(), ws.numel(), stream)
+    if rc in (_lib.ERR_WORKSPACE, _lib.ERR_INVALID):
+        nbytes = lib.kvq_decode_workspace_size(B, Hq, Hkv, L, D, S, 0)
+        if nbytes == 0:
+            raise NotImplementedError(f"decode attention does not support B={B} Hq={Hq} Hkv={Hkv} L={L} D={D} S={S}")
+        if rc == _lib.ERR_WORKSPACE:
+            ws = _workspace(dev, stream, nbytes)
+            rc = fn(*args, ws.data_ptr(), ws.numel(), stream)
+    if rc:
+        _lib.check(rc, symbol)
     return out
 
 

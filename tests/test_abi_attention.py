@@ -219,3 +219,12 @@ def test_narrow_unquantized_head_dims_need_tight_key_rows():
                 "key rows of exactly D")
         _expect(_dense(fn, q=q, out=out, D=80, k=_rows96(1 << 21, 80), v=_rows96(1 << 22, 80)), _lib.ERR_WORKSPACE,
                 "workspace")
+
+
+def test_masked_calls_that_may_take_the_prefill_kernel():
+    """The one rule that the entry point, its workspace size and the lookup of range words go by."""
+    lib = _lib.lib()
+    assert lib.kvq_masked_on_prefill(4, 32, 8, 1023, 128, 1023) == 1
+    for args in ((4, 32, 8, 31, 128, 100000), (1, 8, 8, 128, 128, 3000), (4, 32, 8, 1023, 256, 1023),
+                 (4, 32, 7, 1023, 128, 1023), (0, 32, 8, 1023, 128, 1023)):
+        assert lib.kvq_masked_on_prefill(*args) == 0

@@ -92,6 +92,24 @@ def test_unquantized(D, dtype, kind):
     assert_close(out, ref, f"{kind} D={D}")
 
 
+def test_workspace_too_small():
+    """A masked call that needs more than the stream's workspace gets a larger one and the same results."""
+    B, Hq, Hkv, L, S, D = 1, 8, 2, 200, 3000, 128
+    kt, vt = make_cache(B, Hkv, S, D, 8, torch.float16, 5100)
+    q = seeded_normal((B, Hq, L, D), 5101, torch.float16, DEV)
+    m = left_padded(B, L, S, [77]).to(DEV)
+    ref = kernels.masked_attention(q, kt, vt, 0.1, m, layout="blocked")
+    kernels._workspaces.clear()
+    kernels.masked_attention(q[:, :, :1], kt, vt, 0.1, m[:, :, :1], layout="blocked")
+    small = max(w.numel() for w in kernels._workspaces.values())
+    assert torch.equal(kernels.masked_attention(q, kt, vt, 0.1, m, layout="blocked"), ref)
+    assert max(w.numel() for w in kernels._workspaces.values()) > small
+    with pytest.raises(ValueError):
+        kernels.masked_attention(q, kt, vt, float("nan"), m, layout="blocked")
+    with pytest.raises(NotImplementedError):
+        kernels.masked_attention(q[:, :, :0], kt, vt, 0.1, m[:, :, :0], layout="blocked")
+
+
 def test_mask_and_call_that_stay_on_decode():
     """The same left-padded mask as an additive one over a quantized cache, and into output rows the
     prefill kernel cannot store, give the boolean call's results within two roundings."""
