@@ -55,7 +55,8 @@ DecPlan decode_plan(int B, int Hq, int Hkv, int L, int D, int S, int window, int
   pl.nunits = B * Hkv * pl.rowblocks;
   // as many splits as the target holds whole: a unit count that does not divide 256 would otherwise leave a
   // few workgroups to run after the others. With the count rounded up instead, 32768 8-bit keys of 24, 40
-  // and 72 units took 53.0, 88.7 and 151.9 us; so 41.6, 64.3 and 111.8. Where it costs the workgroups no
+  // and 72 units took 53.0, 88.7 and 151.9 us; so 41.6, 64.3 and 111.8. Past 128 units none is split: 144 and
+  // 240 took 306 and 463 us, so 245 and 371 (5000 keys: 54.7 and 79.2, so 41.6 and 60.5). Where it costs the workgroups no
   // length (or little, and row blocks share keys) the count also makes the grid a multiple of the XCDs,
   // which keeps a unit's splits, and the row blocks of a key range, on one
   auto tiles_of = [&](int n) {

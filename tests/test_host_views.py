@@ -1,5 +1,7 @@
 """The native path's cache views on the CPU: the slices Python would take, and what it hands back."""
 
+import struct
+
 import pytest
 import torch
 
@@ -57,3 +59,12 @@ def test_views_of_a_restored_cache_need_no_library(monkeypatch):
     c.offset = 5
     for tr in c.fetch():
         assert all(torch.equal(a, b[..., :5, :]) for a, b in zip(tr, c.keys))
+
+
+def test_module_has_no_thread_local_storage():
+    """Loaded after torch, a library with a TLS segment slows every thread's access to tensors (see _build.py)."""
+    _lib.host()
+    elf = (_lib.LIB_PATH.parent / "_kvqhost.so").read_bytes()
+    at, size, count = struct.unpack_from("<Q", elf, 32)[0], *struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, at + i * size)[0] for i in range(count)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
